@@ -108,45 +108,13 @@ __device__ __forceinline__ void hiddenOperands(const f32x4 acc[4][4], const floa
 		}
 }
 
-/* In-place bias of a 64 x 64 result tile, and its ReLU packed as the next
- * layer's B operand (pack without ReLU for gradients). */
-__device__ __forceinline__ void biasInPlace(f32x4 acc[4][4], const float* bias, int g)
-{
-#pragma unroll
-	for (int mb = 0; mb < 4; mb++)
-#pragma unroll
-		for (int r = 0; r < 4; r++)
-		{
-			const float b = bias[16 * mb + 4 * g + r];
-#pragma unroll
-			for (int nb = 0; nb < 4; nb++)
-				acc[mb][nb][r] += b;
-		}
-}
-
-template <bool RELU>
-__device__ __forceinline__ void packOperands(const f32x4 acc[4][4], bf16x8 h[2][4])
-{
-#pragma unroll
-	for (int mb = 0; mb < 4; mb++)
-#pragma unroll
-		for (int r = 0; r < 4; r++)
-#pragma unroll
-			for (int nb = 0; nb < 4; nb++)
-			{
-				const float v = acc[mb][nb][r];
-				h[mb >> 1][nb][4 * (mb & 1) + r] = (__bf16) (RELU ? (v > 0.0f ? v : 0.0f) : v);
-			}
-}
-
 /* Layer 1 for the wave's 64 fragments: acc[mb][nb] = W1 X^T (no bias).
  * xin = this lane's own fragment's features, step = the network's
  * frequency steps; column 16nb + c of X^T is lane 16nb + c's fragment,
  * fetched by shuffle one feature at a time (so no lane holds all four
- * columns' features at once).  If xt != nullptr the encoded operand is also
- * stored transposed (xt[k * ld + col0 + 16nb + c]). */
+ * columns' features at once). */
 __device__ __forceinline__ void layer1(const uint16_t* __restrict__ w1, const float* step, const float xin[SRP_NN_IN],
-                                       int g, int c, f32x4 acc[4][4], __bf16* xt = nullptr, size_t ld = 0)
+                                       int g, int c, f32x4 acc[4][4])
 {
 #pragma unroll
 	for (int mb = 0; mb < 4; mb++)
@@ -177,13 +145,7 @@ __device__ __forceinline__ void layer1(const uint16_t* __restrict__ w1, const fl
 			bf16x8 b[4];
 #pragma unroll
 			for (int nb = 0; nb < 4; nb++)
-			{
 				b[nb] = encode8(ud[nb], j0, sd[nb], cd[nb]);
-				if (xt)
-#pragma unroll
-					for (int q = 0; q < 8; q++)
-						xt[(size_t) (32 * ks + 8 * g + q) * ld + 16 * nb + c] = b[nb][q];
-			}
 #pragma unroll
 			for (int mb = 0; mb < 4; mb++)
 			{
