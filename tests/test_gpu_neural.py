@@ -373,3 +373,27 @@ def test_neural_shader_end_to_end(nn):
 def no_rgb(color):
     from neural_runner import rgb_of
     return rgb_of(color)
+
+
+@pytest.mark.parametrize("chunks", [1, 9])
+def test_gradients_match_oracle_across_chunk_counts(nn, chunks):
+    """One 1,024-sample chunk, and nine (a whole group of eight partial sums
+    and a remainder, chunks that do not divide by the XCDs): each tensor's
+    gradient within the bf16 operands' rounding of the oracle's."""
+    n = 1024 * chunks
+    F, T = synth(n, 40 + chunks)
+    ds = nn.new_ds(n)
+    net = nn.new_net(6)
+    try:
+        nn.ds_write(ds, F, T)
+        p = (no.init_params(6) * 3.0).astype(np.float32)
+        nn.set_params(net, p)
+        g, loss = nn.gradients(net, ds, n)
+        lo, go = no.loss_and_grad(p.astype(np.float64), F, T, bf=True)
+        assert abs(loss - lo) <= 1e-4 * lo
+        for a, b in ((no.OFF_W1, no.OFF_B1), (no.OFF_B1, no.OFF_W2), (no.OFF_W2, no.OFF_B2), (no.OFF_B2, no.OFF_W3),
+                     (no.OFF_W3, no.OFF_B3), (no.OFF_B3, no.N_PARAMS)):
+            assert np.linalg.norm(g[a:b] - go[a:b]) <= 1e-2 * np.linalg.norm(go[a:b])
+    finally:
+        nn.free_net(net)
+        nn.free_ds(ds)
