@@ -30,3 +30,33 @@
 #else
 #  define SRP_INLINE_MATH 0
 #endif
+
+/* Device code: a generic pointer known to point to global memory, and one
+ * to global memory that nothing writes while the kernel runs.  A pointer
+ * read from memory has no known address space: loads through it are flat
+ * (and wait for LDS traffic too), and a wave-uniform load that some store of
+ * the kernel might alias goes through the vector memory path, several
+ * hundred cycles each, instead of the scalar cache.  Casting to the address
+ * space and back tells the compiler (by way of an integer: a direct pair of
+ * casts is folded away); the pointer itself is unchanged. */
+#if defined(__HIPCC__)
+#include <stdint.h>
+template <class T>
+__host__ __device__ inline __attribute__((always_inline)) T* srpGlobal(T* p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+	return (T*) (__attribute__((address_space(1))) T*) (uintptr_t) p;
+#else
+	return p;
+#endif
+}
+template <class T>
+__host__ __device__ inline __attribute__((always_inline)) const T* srpConst(const T* p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+	return (const T*) (const __attribute__((address_space(4))) T*) (uintptr_t) p;
+#else
+	return p;
+#endif
+}
+#endif

@@ -18,7 +18,7 @@ SRP_EXTERN_C_END
 static inline __host__ __device__ void srpTextureGetFilteredColor(const SRPTexture* tex, float u, float v, float out[4])
 {
 #if defined(__HIP_DEVICE_COMPILE__)
-	const SrpTexDesc* d = (const SrpTexDesc*) tex;
+	const SrpTexDesc* d = srpConst((const SrpTexDesc*) tex);
 	if (u < 0 || u > 1)
 		u = (d->wrapX == TW_REPEAT) ? (float) ((double) u - floor((double) u)) : (float) fmax(0.0, fmin(1.0, (double) u));
 	if (v < 0 || v > 1)
@@ -26,11 +26,12 @@ static inline __host__ __device__ void srpTextureGetFilteredColor(const SRPTextu
 	const float x = (float) d->wM1 * u;
 	const float y = (float) d->hM1 * (1 - v);
 	const double xd = (double) x + 0.5, yd = (double) y + 0.5;
-	int64_t xi = (xd >= 0.0 && xd < 9.0e18) ? (int64_t) xd : 0;
-	int64_t yi = (yd >= 0.0 && yd < 9.0e18) ? (int64_t) yd : 0;
-	if (xi > d->wM1) xi = d->wM1;
-	if (yi > d->hM1) yi = d->hM1;
-	const uint32_t texel = d->texels[yi * (int64_t) d->w + xi];
+	/* u and v lie in [0, 1] or are NaN, so the coordinates are below 2^32 */
+	uint32_t xi = (xd >= 0.0 && xd < 4294967296.0) ? (uint32_t) xd : 0u;
+	uint32_t yi = (yd >= 0.0 && yd < 4294967296.0) ? (uint32_t) yd : 0u;
+	if (xi > (uint32_t) d->wM1) xi = (uint32_t) d->wM1;
+	if (yi > (uint32_t) d->hM1) yi = (uint32_t) d->hM1;
+	const uint32_t texel = srpGlobal(d->texels)[(uint64_t) yi * (uint32_t) d->w + xi];
 	const float inv255 = (float) (1. / 255.);
 	out[0] = (float) (int) (texel & 255u) * inv255;
 	out[1] = (float) (int) ((texel >> 8) & 255u) * inv255;

@@ -11,7 +11,7 @@
 #include <stdint.h>
 #include "srp/context.h"
 
-#define SRP_ABI_VERSION 16u
+#define SRP_ABI_VERSION 17u
 #define SRP_MAX_VARYINGS 16
 #define SRP_MAX_WORDS 32          /* fast interpolation path: 4-byte words */
 #define SRP_MAX_VARYING_BYTES 256 /* general path: bytes per fragment */
@@ -32,15 +32,6 @@
 #define SRP_EDGE_TL_THRESHOLD (-0x1.12e0c0p-30f)
 #define SRP_STAT_SLOTS 64
 #define SRP_STAT_STRIDE 16
-
-/* interpolation kinds of a 4-byte word in the fast path */
-enum SrpWordKind
-{
-	SRP_WORD_PERSPECTIVE = 0,  /* float, perspective-correct */
-	SRP_WORD_AFFINE = 1,       /* float, screen-space linear */
-	SRP_WORD_PROVOKING = 2,    /* flat float or integer bytes: provoking vertex */
-	SRP_WORD_UNUSED = 3        /* padding beyond the described varyings */
-};
 
 typedef struct SrpVaryingDesc
 {
@@ -137,7 +128,9 @@ typedef struct SrpDrawParams
 	SrpVaryingDesc var[SRP_MAX_VARYINGS];
 	uint32_t wordPath;       /* 1: every element 4-byte and aligned */
 	uint32_t nWords;
-	uint8_t wordKind[SRP_MAX_WORDS];
+	/* how word k interpolates (bit k; in none of them: zero): perspective,
+	 * affine, or copied from the provoking vertex (flat and integer) */
+	uint32_t wordPerspective, wordAffine, wordProvoking;
 
 	/* tiles */
 	uint32_t tileShift, tilesX, tilesY;

@@ -15,6 +15,7 @@
 #include <stdint.h>
 
 #include "srp/neural_abi.h"
+#include "srp/detail/qualifiers.h"
 
 namespace srp {
 namespace nn {
@@ -216,17 +217,21 @@ __device__ inline void inferWave(const SrpNnDevice* __restrict__ net, const floa
 {
 	const int lane = (int) (threadIdx.x & 63u);
 	const int g = lane >> 4, c = lane & 15;
+	/* the network does not change while it is evaluated, and lies in global
+	 * memory; the pointers to it come from memory, so say so */
+	net = srpConst((const SrpNnDevice*) net);
 	f32x4 acc[4][4];
-	layer1(net->w1, net->step, xin, g, c, acc);
+	layer1(srpGlobal(net->w1), net->step, xin, g, c, acc);
 	bf16x8 h[2][4];
-	hiddenOperands(acc, net->b1, g, h);
-	layerHidden(net->w2f, h, g, c, acc);
-	hiddenOperands(acc, net->b2, g, h);
+	hiddenOperands(acc, srpGlobal(net->b1), g, h);
+	layerHidden(srpGlobal(net->w2f), h, g, c, acc);
+	hiddenOperands(acc, srpGlobal(net->b2), g, h);
 	f32x4 y[4];
-	layerOut(net->w3f, h, g, c, y);
+	layerOut(srpGlobal(net->w3f), h, g, c, y);
+	const float* b3 = srpConst(net->b3);
 #pragma unroll
 	for (int ch = 0; ch < 3; ch++)
-		rgb[ch] = ownOutput(y, ch, lane) + net->b3[ch];
+		rgb[ch] = ownOutput(y, ch, lane) + b3[ch];
 }
 
 __device__ __forceinline__ float bf(uint16_t bits)

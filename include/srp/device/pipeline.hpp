@@ -69,7 +69,21 @@ __device__ __forceinline__ bool compare(uint32_t op, T lhs, T rhs)
 }
 
 /* reference raster/fragment.c:180-223: op result merged under the write mask */
-__device__ __forceinline__ uint32_t stencilApply(uint32_t op, uint32_t s, const SRPStencilFaceState& st)
+struct FaceState
+{
+	uint32_t func, ref, mask, writeMask, sfailOp, dfailOp, passOp;
+};
+/* One face's stencil state, read as words: its byte fields would each be a
+ * vector memory load (the scalar loads have no byte form). */
+__device__ __forceinline__ FaceState faceState(const SrpState& st, int face)
+{
+	static_assert(sizeof(SRPStencilFaceState) == 20, "func; ref, mask, writeMask; the three ops");
+	uint32_t w[5];
+	__builtin_memcpy(w, &st.stencil[face], 20);
+	return FaceState{w[0], w[1] & 255u, (w[1] >> 8) & 255u, (w[1] >> 16) & 255u, w[2], w[3], w[4]};
+}
+
+__device__ __forceinline__ uint32_t stencilApply(uint32_t op, uint32_t s, const FaceState& st)
 {
 	uint32_t v;
 	switch (op)
@@ -115,8 +129,8 @@ __device__ __forceinline__ float replay(float a, float d, int n)
 /* Varying bytes of a vertex slot: post-VS cache or clip-generated vertex. */
 __device__ __forceinline__ const uint8_t* varyingPtr(const SrpDrawParams* P, uint32_t vref)
 {
-	return (vref < P->cacheSize) ? P->varyings + (size_t) vref * P->varyingsSize
-	                             : P->genVaryings + (size_t) (vref - P->cacheSize) * P->varyingsSize;
+	return srpGlobal((vref < P->cacheSize) ? P->varyings + (size_t) vref * P->varyingsSize
+	                                       : P->genVaryings + (size_t) (vref - P->cacheSize) * P->varyingsSize);
 }
 
 __device__ __forceinline__ float loadF(const uint8_t* p)
@@ -154,36 +168,49 @@ template <int N>
 __device__ __forceinline__ void interpWords(const SrpDrawParams* P, const uint32_t* const* v, const float* w,
                                             const float* invW, float rec, uint32_t pv, uint32_t* out)
 {
+	const uint32_t nWords = P->nWords;
+	const uint32_t persp = P->wordPerspective, affine = P->wordAffine, copied = P->wordProvoking;
+	/* four words of every vertex at a time, requested before any is used
+	 * (the varying buffers end in 512 spare bytes, so the last four may reach
+	 * past the words described) */
 #pragma unroll
-	for (int k = 0; k < SRP_MAX_WORDS; k++)
+	for (int k0 = 0; k0 < SRP_MAX_WORDS; k0 += 4)
 	{
-		if (k >= (int) P->nWords)
+		if (k0 >= (int) nWords)
 		{
-			out[k] = 0u;
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+				out[k0 + q] = 0u;
 			continue;
 		}
-		const uint32_t kind = P->wordKind[k];
-		if (kind == SRP_WORD_PERSPECTIVE)
-		{
-			float val = 0.0f;
+		uint32_t a[N][4];
 #pragma unroll
-			for (int i = 0; i < N; i++)
-				val += __uint_as_float(v[i][k]) * invW[i] * w[i];
-			val *= rec;
-			out[k] = __float_as_uint(val);
-		}
-		else if (kind == SRP_WORD_AFFINE)
-		{
-			float val = 0.0f;
+		for (int i = 0; i < N; i++)
+			__builtin_memcpy(a[i], v[i] + k0, 16);
 #pragma unroll
-			for (int i = 0; i < N; i++)
-				val += __uint_as_float(v[i][k]) * w[i];
-			out[k] = __float_as_uint(val);
+		for (int q = 0; q < 4; q++)
+		{
+			const int k = k0 + q;
+			if ((persp >> k) & 1u)
+			{
+				float val = 0.0f;
+#pragma unroll
+				for (int i = 0; i < N; i++)
+					val += __uint_as_float(a[i][q]) * invW[i] * w[i];
+				val *= rec;
+				out[k] = __float_as_uint(val);
+			}
+			else if ((affine >> k) & 1u)
+			{
+				float val = 0.0f;
+#pragma unroll
+				for (int i = 0; i < N; i++)
+					val += __uint_as_float(a[i][q]) * w[i];
+				out[k] = __float_as_uint(val);
+			}
+			else
+				out[k] = ((copied >> k) & 1u) ? (pv ? a[N - 1][q] : a[0][q]) : 0u;
 		}
-		else if (kind == SRP_WORD_PROVOKING)
-			out[k] = v[pv][k];
-		else
-			out[k] = 0u;
 	}
 }
 
@@ -268,9 +295,11 @@ __device__ __forceinline__ void fragment(const SrpDrawParams* P, int px, int py,
 		if (ux < st.sx0 || ux >= st.sx1 || uy < st.sy0 || uy >= st.sy1)
 			return;
 	}
-	const SRPStencilFaceState& sf = st.stencil[front ? 0 : 1];
+	FaceState sf = {};
+	if (st.stencilEnabled)
+		sf = faceState(st, front ? 0 : 1);
 	const float stored = ps.depth;
-	if (st.stencilEnabled && !compare<uint32_t>(sf.func, (uint32_t) (sf.ref & sf.mask), ps.stencil & sf.mask))
+	if (st.stencilEnabled && !compare<uint32_t>(sf.func, sf.ref & sf.mask, ps.stencil & sf.mask))
 	{
 		ps.stencil = stencilApply(sf.sfailOp, ps.stencil, sf);
 		return;
@@ -281,7 +310,7 @@ __device__ __forceinline__ void fragment(const SrpDrawParams* P, int px, int py,
 		return;
 	}
 	SRPFragmentShaderIn in;
-	in.uniform = (SRPUniform*) P->uniform;
+	in.uniform = (SRPUniform*) srpGlobal(P->uniform);
 	in.fragCoord[0] = (float) ((double) px + 0.5);
 	in.fragCoord[1] = (float) ((double) py + 0.5);
 	in.fragCoord[2] = depth;
@@ -319,7 +348,7 @@ __device__ __forceinline__ void flushStats(const SrpDrawParams* P, uint32_t cove
 	}
 	if ((threadIdx.x & 63) == 0 && (covered | shaded))
 	{
-		unsigned long long* c = P->stats + (size_t) (blockIdx.x % SRP_STAT_SLOTS) * SRP_STAT_STRIDE;
+		unsigned long long* c = srpGlobal(P->stats) + (size_t) (blockIdx.x % SRP_STAT_SLOTS) * SRP_STAT_STRIDE;
 		atomicAdd(&c[0], (unsigned long long) covered);
 		atomicAdd(&c[1], (unsigned long long) shaded);
 	}
@@ -369,38 +398,39 @@ __global__ __launch_bounds__(256) void srp_vs_kernel(SrpVsLaunch L)
 		fillBlock(L, blockIdx.x - vsBlocks);
 		return;
 	}
-	const SrpDrawParams* P = L.params;
+	const SrpDrawParams* P = srpConst(L.params);
 	uint32_t i = blockIdx.x * 256u + threadIdx.x;
 	uint32_t count = L.count;
 	if (L.nSeg)
 	{
+		const SrpSeg* seg = srpConst(L.seg);
 		uint32_t a = 0, b = L.nSeg;
 		while (b - a > 1)
 		{
 			const uint32_t m = (a + b) >> 1;
-			if (L.seg[m].firstBlock <= blockIdx.x) a = m;
+			if (seg[m].firstBlock <= blockIdx.x) a = m;
 			else b = m;
 		}
-		P = L.seg[a].P;
-		i = (blockIdx.x - L.seg[a].firstBlock) * 256u + threadIdx.x;
-		count = L.seg[a].count;
+		P = srpConst(seg[a].P);
+		i = (blockIdx.x - seg[a].firstBlock) * 256u + threadIdx.x;
+		count = seg[a].count;
 	}
 	if (i >= count)
 		return;
 	const uint64_t vi = P->cacheBase + i;
 	SRPVertexShaderIn in;
-	in.uniform = (SRPUniform*) P->uniform;
-	in.vertex = (SRPVertex*) (P->vertices + vi * P->vertexStride);
+	in.uniform = (SRPUniform*) srpGlobal(P->uniform);
+	in.vertex = (SRPVertex*) srpGlobal(P->vertices + vi * P->vertexStride);
 	in.vertexID = (size_t) vi;
 	SRPVertexShaderOut out;
 	out.clipPosition[0] = 0.0f; out.clipPosition[1] = 0.0f;
 	out.clipPosition[2] = 0.0f; out.clipPosition[3] = 0.0f;
-	out.varyings = (SRPVarying*) (P->varyings + (size_t) i * P->varyingsSize);
+	out.varyings = (SRPVarying*) srpGlobal(P->varyings + (size_t) i * P->varyingsSize);
 	VS()(&in, &out);
 	float4 c;
 	c.x = out.clipPosition[0]; c.y = out.clipPosition[1];
 	c.z = out.clipPosition[2]; c.w = out.clipPosition[3];
-	reinterpret_cast<float4*>(P->clip)[i] = c;
+	srpGlobal(reinterpret_cast<float4*>(P->clip))[i] = c;
 }
 
 /* Blocks are issued round-robin over the 8 XCDs (block b to XCD b % 8).
@@ -454,9 +484,9 @@ __device__ __forceinline__ void rasterTileSimple(const SrpRasterLaunch& L, const
 	ps.color = 0; ps.depth = 0.0f; ps.stencil = 0; ps.covered = 0; ps.shaded = 0;
 	if (inFb)
 	{
-		ps.color = P->color[idx];
-		ps.depth = P->depth[idx];
-		ps.stencil = P->stencil[idx];
+		ps.color = srpGlobal(P->color)[idx];
+		ps.depth = srpGlobal(P->depth)[idx];
+		ps.stencil = srpGlobal(P->stencil)[idx];
 	}
 	const uint32_t pv = P->st.provokingLast ? 2u : 0u;
 
@@ -506,9 +536,9 @@ __device__ __forceinline__ void rasterTileSimple(const SrpRasterLaunch& L, const
 	}
 	if (inFb)
 	{
-		P->color[idx] = ps.color;
-		P->depth[idx] = ps.depth;
-		P->stencil[idx] = (uint8_t) ps.stencil;
+		srpGlobal(P->color)[idx] = ps.color;
+		srpGlobal(P->depth)[idx] = ps.depth;
+		srpGlobal(P->stencil)[idx] = (uint8_t) ps.stencil;
 	}
 	covered += ps.covered;
 	shaded += ps.shaded;
@@ -524,7 +554,7 @@ __global__ __launch_bounds__(256) void srp_raster_kernel(SrpRasterLaunch L)
 	if (tile >= L.nTiles)
 		return;
 	uint32_t covered = 0, shaded = 0;
-	rasterTileSimple<FS, LATE, WORDS, TILE>(L, L.params, tile, tile, local, covered, shaded);
+	rasterTileSimple<FS, LATE, WORDS, TILE>(L, srpConst(L.params), tile, tile, local, covered, shaded);
 	flushStats(L.params, covered, shaded);
 }
 
@@ -540,6 +570,7 @@ __global__ __launch_bounds__(256) void srp_raster_persistent16(SrpRasterLaunch L
 	const uint32_t q0 = blockIdx.x % nq;
 	uint32_t covered = 0, shaded = 0;
 	const SrpDrawParams* last = nullptr;
+	const SrpSeg* seg = srpConst(L.seg);
 	for (uint32_t k = 0; k < nq; k++)
 	{
 		const uint32_t q = (q0 + k) % nq;
@@ -558,11 +589,11 @@ __global__ __launch_bounds__(256) void srp_raster_persistent16(SrpRasterLaunch L
 			while (b - a > 1)
 			{
 				const uint32_t m = (a + b) >> 1;
-				if (L.seg[m].first <= t) a = m;
+				if (seg[m].first <= t) a = m;
 				else b = m;
 			}
-			const SrpSeg sg = L.seg[a];
-			rasterTileSimple<FS, LATE, WORDS, 16>(L, sg.P, t - sg.first, t, threadIdx.x, covered, shaded);
+			const SrpSeg sg = seg[a];
+			rasterTileSimple<FS, LATE, WORDS, 16>(L, srpConst(sg.P), t - sg.first, t, threadIdx.x, covered, shaded);
 			last = sg.P;
 		}
 	}
@@ -746,11 +777,17 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 	bool wrote = false;   /* DEFER: the draw wrote this pixel's colour */
 	if (inFb)
 	{
-		col = P->color[idx];
-		dep = P->depth[idx];
-		sten = P->stencil[idx];
+		col = srpGlobal(P->color)[idx];
+		dep = srpGlobal(P->depth)[idx];
+		sten = srpGlobal(P->stencil)[idx];
 	}
 	const uint32_t pv = st.provokingLast ? 2u : 0u;
+	FaceState face0 = {}, face1 = {};
+	if (st.stencilEnabled)
+	{
+		face0 = faceState(st, 0);
+		face1 = faceState(st, 1);
+	}
 	const bool precull = !LATE && st.depthTest && monotoneOp(st.depthOp);
 	/* whole-tile depth culling of pixel-parallel runs: a culled fragment
 	 * must have no effect at all, so no stencil (its dfail op) and no
@@ -873,7 +910,7 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 					cov = insideTri(T, l);
 				}
 				const bool front = (T.flags >> 3) & 1u;
-				const SRPStencilFaceState& sf = st.stencil[front ? 0 : 1];
+				const FaceState sf = front ? face0 : face1;
 				const float iw[3] = {T.invW[0], T.invW[1], T.invW[2]};
 				float depth = 0.0f, rec = 0.0f;
 				bool active = false;
@@ -890,7 +927,7 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 							active = false;
 					}
 					if (active && st.stencilEnabled &&
-					    !compare<uint32_t>(sf.func, (uint32_t) (sf.ref & sf.mask), sten & sf.mask))
+					    !compare<uint32_t>(sf.func, sf.ref & sf.mask, sten & sf.mask))
 					{
 						sten = stencilApply(sf.sfailOp, sten, sf);
 						active = false;
@@ -908,7 +945,7 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 				typedef typename VaryingBuf<WORDS>::type BufT;
 				BufT buf[VaryingBuf<WORDS>::n];
 				in.varyings = (SRPInterpolated*) buf;
-				in.uniform = (SRPUniform*) P->uniform;
+				in.uniform = (SRPUniform*) srpGlobal(P->uniform);
 				in.fragCoord[0] = (float) ((double) px + 0.5);
 				in.fragCoord[1] = (float) ((double) py + 0.5);
 				in.fragCoord[2] = depth;
@@ -1085,7 +1122,7 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 					state = FRAG_CULLED;
 				if (state == FRAG_SHADED && !DEFER)
 				{
-					in.uniform = (SRPUniform*) P->uniform;
+					in.uniform = (SRPUniform*) srpGlobal(P->uniform);
 					in.fragCoord[0] = (float) ((double) fx + 0.5);
 					in.fragCoord[1] = (float) ((double) fy + 0.5);
 					in.fragCoord[2] = depth;
@@ -1119,7 +1156,7 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 				/* every lane calls; lanes without a fragment pass zeroed inputs */
 				if (!active)
 				{
-					in.uniform = (SRPUniform*) P->uniform;
+					in.uniform = (SRPUniform*) srpGlobal(P->uniform);
 					in.fragCoord[0] = 0.0f; in.fragCoord[1] = 0.0f; in.fragCoord[2] = 0.0f; in.fragCoord[3] = 0.0f;
 					in.frontFacing = 0;
 					in.primitiveID = 0;
@@ -1157,8 +1194,8 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 			if (state == FRAG_SCISSORED)
 				continue;
 			const bool front = (fragState[f] & FRAG_FRONT) != 0;
-			const SRPStencilFaceState& sf = st.stencil[front ? 0 : 1];
-			if (st.stencilEnabled && !compare<uint32_t>(sf.func, (uint32_t) (sf.ref & sf.mask), sten & sf.mask))
+			const FaceState sf = front ? face0 : face1;
+			if (st.stencilEnabled && !compare<uint32_t>(sf.func, sf.ref & sf.mask, sten & sf.mask))
 			{
 				sten = stencilApply(sf.sfailOp, sten, sf);
 				continue;
@@ -1188,9 +1225,9 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 	if (inFb)
 	{
 		if (!DEFER)
-			P->color[idx] = col;
-		P->depth[idx] = dep;
-		P->stencil[idx] = (uint8_t) sten;
+			srpGlobal(P->color)[idx] = col;
+		srpGlobal(P->depth)[idx] = dep;
+		srpGlobal(P->stencil)[idx] = (uint8_t) sten;
 	}
 	if (DEFER)
 	{
@@ -1215,7 +1252,7 @@ __global__ __launch_bounds__(64, WAVES) void srp_raster_batched(SrpRasterLaunch 
 	if (tile >= L.nTiles)
 		return;
 	uint32_t covered = 0, shaded = 0;
-	rasterTileBatched<FS, LATE, WORDS, CULL, DEFER>(L, L.params, tile, tile, covered, shaded);
+	rasterTileBatched<FS, LATE, WORDS, CULL, DEFER>(L, srpConst(L.params), tile, tile, covered, shaded);
 	flushStats(L.params, covered, shaded);
 }
 
@@ -1238,7 +1275,7 @@ __device__ __forceinline__ uint32_t deferWords(const SrpDrawParams* P, bool word
 template <bool WORDS>
 __global__ __launch_bounds__(256) void srp_defer_gather(SrpRasterLaunch L)
 {
-	const SrpDrawParams* P = L.params;
+	const SrpDrawParams* P = srpConst(L.params);
 	const uint32_t pv = P->st.provokingLast ? 2u : 0u;
 	const uint32_t width = P->width;
 	const size_t S = L.deferStride;
@@ -1294,7 +1331,7 @@ __global__ __launch_bounds__(256) void srp_defer_gather(SrpRasterLaunch L)
 template <class FS, bool WORDS>
 __global__ __launch_bounds__(256, 2) void srp_defer_shade(SrpRasterLaunch L)
 {
-	const SrpDrawParams* P = L.params;
+	const SrpDrawParams* P = srpConst(L.params);
 	const uint32_t n = L.deferCounts[L.nTiles];
 	const uint32_t lane = threadIdx.x & 63u;
 	const size_t S = L.deferStride;
@@ -1313,7 +1350,7 @@ __global__ __launch_bounds__(256, 2) void srp_defer_shade(SrpRasterLaunch L)
 		for (uint32_t q = 0; q < VaryingBuf<WORDS>::n; q++)
 			buf[q] = (active && q < nw) ? F[(7 + q) * S + k] : 0u;
 		in.varyings = (SRPInterpolated*) buf;
-		in.uniform = (SRPUniform*) P->uniform;
+		in.uniform = (SRPUniform*) srpGlobal(P->uniform);
 		in.fragCoord[0] = active ? __uint_as_float(F[0 * S + k]) : 0.0f;
 		in.fragCoord[1] = active ? __uint_as_float(F[1 * S + k]) : 0.0f;
 		in.fragCoord[2] = active ? __uint_as_float(F[2 * S + k]) : 0.0f;
@@ -1322,7 +1359,7 @@ __global__ __launch_bounds__(256, 2) void srp_defer_shade(SrpRasterLaunch L)
 		in.primitiveID = active ? F[5 * S + k] : 0u;
 		FS().wave(&in, &out, active);
 		if (active)
-			P->color[F[6 * S + k]] = packColor(out.color);
+			srpGlobal(P->color)[F[6 * S + k]] = packColor(out.color);
 	}
 }
 
@@ -1339,6 +1376,7 @@ __global__ __launch_bounds__(64, WAVES) void srp_raster_persistent(SrpRasterLaun
 	const uint32_t q0 = blockIdx.x % nq;
 	uint32_t covered = 0, shaded = 0;
 	const SrpDrawParams* last = nullptr;
+	const SrpSeg* seg = srpConst(L.seg);
 	for (uint32_t k = 0; k < nq; k++)
 	{
 		const uint32_t q = (q0 + k) % nq;
@@ -1357,11 +1395,11 @@ __global__ __launch_bounds__(64, WAVES) void srp_raster_persistent(SrpRasterLaun
 			while (b - a > 1)
 			{
 				const uint32_t m = (a + b) >> 1;
-				if (L.seg[m].first <= t) a = m;
+				if (seg[m].first <= t) a = m;
 				else b = m;
 			}
-			const SrpSeg sg = L.seg[a];
-			rasterTileBatched<FS, LATE, WORDS, CULL>(L, sg.P, t - sg.first, t, covered, shaded);
+			const SrpSeg sg = seg[a];
+			rasterTileBatched<FS, LATE, WORDS, CULL>(L, srpConst(sg.P), t - sg.first, t, covered, shaded);
 			last = sg.P;
 		}
 	}
@@ -1376,7 +1414,7 @@ template <class FS, bool LATE, bool WORDS>
 __global__ __launch_bounds__(256) void srp_frag_kernel(SrpFragLaunch L)
 {
 	const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-	const SrpDrawParams* P = L.params;
+	const SrpDrawParams* P = srpConst(L.params);
 	PixelState ps;
 	ps.color = 0; ps.depth = 0.0f; ps.stencil = 0; ps.covered = 0; ps.shaded = 0;
 	const uint32_t npix = P->width * P->height;
@@ -1392,9 +1430,9 @@ __global__ __launch_bounds__(256) void srp_frag_kernel(SrpFragLaunch L)
 	}
 	if (head)
 	{
-		ps.color = P->color[key];
-		ps.depth = P->depth[key];
-		ps.stencil = P->stencil[key];
+		ps.color = srpGlobal(P->color)[key];
+		ps.depth = srpGlobal(P->depth)[key];
+		ps.stencil = srpGlobal(P->stencil)[key];
 		const uint32_t pv = P->st.provokingLast ? 1u : 0u;
 		for (uint32_t j = i; j < count && L.keys[j] == key; j++)
 		{
@@ -1438,9 +1476,9 @@ __global__ __launch_bounds__(256) void srp_frag_kernel(SrpFragLaunch L)
 				});
 			}
 		}
-		P->color[key] = ps.color;
-		P->depth[key] = ps.depth;
-		P->stencil[key] = (uint8_t) ps.stencil;
+		srpGlobal(P->color)[key] = ps.color;
+		srpGlobal(P->depth)[key] = ps.depth;
+		srpGlobal(P->stencil)[key] = (uint8_t) ps.stencil;
 	}
 	flushStats(P, ps.covered, ps.shaded);
 }

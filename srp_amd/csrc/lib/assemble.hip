@@ -85,9 +85,10 @@ __device__ __forceinline__ uint64_t loadIndex(const uint8_t* ib, uint32_t elem, 
 
 __device__ __forceinline__ uint32_t slotOf(const AsmDraw& W, uint64_t stream)
 {
-	const uint64_t vi = W.indexElem ? loadIndex(W.indices, W.indexElem, stream) : stream;
-	const uint64_t slot = vi - W.P->cacheBase;
-	return slot < (uint64_t) W.P->cacheSize ? (uint32_t) slot : 0xFFFFFFFFu;
+	const SrpDrawParams* P = srpConst(W.P);
+	const uint64_t vi = W.indexElem ? loadIndex(srpGlobal(W.indices), W.indexElem, stream) : stream;
+	const uint64_t slot = vi - P->cacheBase;
+	return slot < (uint64_t) P->cacheSize ? (uint32_t) slot : 0xFFFFFFFFu;
 }
 
 /* A vertex index outside the range the draw's post-VS cache was prepared
@@ -120,7 +121,7 @@ __device__ __forceinline__ uint32_t drawOfBlock(const AsmDraw* D, uint32_t n, ui
 
 __device__ __forceinline__ void loadClip(const SrpDrawParams* P, uint32_t slot, float* c)
 {
-	const float4 v = reinterpret_cast<const float4*>(P->clip)[slot];
+	const float4 v = srpGlobal(reinterpret_cast<const float4*>(P->clip))[slot];
 	c[0] = v.x; c[1] = v.y; c[2] = v.z; c[3] = v.w;
 }
 
@@ -424,7 +425,7 @@ __device__ void emitLineFrags(const AsmArgs& A, const SrpDrawParams* P, const Sr
 		x += xInc; y += yInc; t += tInc;
 	}
 	if (invalid)
-		atomicAdd(&P->stats[(size_t) (blockIdx.x % SRP_STAT_SLOTS) * SRP_STAT_STRIDE], (unsigned long long) invalid);
+		atomicAdd(&srpGlobal(P->stats)[(size_t) (blockIdx.x % SRP_STAT_SLOTS) * SRP_STAT_STRIDE], (unsigned long long) invalid);
 }
 
 /* point.c:81-118: pixel bounds of a point; false when fully outside. */
@@ -511,7 +512,7 @@ __device__ __forceinline__ void fanTriangle(const AsmArgs& A, const AsmDraw& W, 
                                             uint32_t recBase, uint32_t idBase, uint32_t itemBase, uint32_t& nRec,
                                             uint32_t& nItems, bool drop)
 {
-	const SrpDrawParams* P = W.P;
+	const SrpDrawParams* P = srpConst(W.P);
 	const uint32_t mode = P->st.polygonMode;
 	if (mode == SRP_POLYGON_MODE_FILL)
 	{
@@ -639,13 +640,13 @@ __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 	if (!EMIT && A.zero)
 		for (uint32_t z = blockIdx.x * 128u + threadIdx.x; z < A.zeroCount; z += gridDim.x * 128u)
 			A.zero[z] = 0u;
-	const uint32_t d = A.nDraws > 1 ? drawOfBlock(A.draws, A.nDraws, blockIdx.x) : 0u;
-	const AsmDraw& W = A.draws[d];
+	const uint32_t d = A.nDraws > 1 ? drawOfBlock(srpConst(A.draws), A.nDraws, blockIdx.x) : 0u;
+	const AsmDraw& W = srpConst(A.draws)[d];
 	const uint32_t k = (blockIdx.x - W.firstBlock) * 128u + threadIdx.x;
 	if (k >= W.nIn)
 		return;
 	const uint32_t g = W.primBase + k;   /* slot of this input in the count arrays */
-	const SrpDrawParams* P = W.P;
+	const SrpDrawParams* P = srpConst(W.P);
 	uint64_t s[3];
 	triStream(W.prim, W.start, k, s);
 	uint32_t slot[3];
@@ -750,7 +751,7 @@ __device__ __forceinline__ void clipFillFans(const AsmArgs& A, const AsmDraw& W,
                                              const Vtx& b, const Vtx& c, bool fan, uint32_t recBase, uint32_t idBase,
                                              uint32_t itemBase, bool drop)
 {
-	const SrpDrawParams* P = W.P;
+	const SrpDrawParams* P = srpConst(W.P);
 	SrpTri T = {};
 	const bool ok = fan && setupTriangle(P, a, b, c, 0u, T);
 	const bool span = ok && isSpan(P, T);
@@ -925,9 +926,9 @@ __device__ __forceinline__ void clipFillFans(const AsmArgs& A, const AsmDraw& W,
 template <bool EMIT>
 __device__ __forceinline__ void clipGroup(const AsmArgs& A, uint32_t g, bool has, uint32_t gl)
 {
-	const uint32_t d = (has && A.nDraws > 1) ? drawOfInput(A.draws, A.nDraws, g) : 0u;
-	const AsmDraw& W = A.draws[d];
-	const SrpDrawParams* P = W.P;
+	const uint32_t d = (has && A.nDraws > 1) ? drawOfInput(srpConst(A.draws), A.nDraws, g) : 0u;
+	const AsmDraw& W = srpConst(A.draws)[d];
+	const SrpDrawParams* P = srpConst(W.P);
 	const uint32_t gshift = __lane_id() & ~(CLIP_GROUP - 1u);
 	const uint64_t below = (1ull << gl) - 1ull;
 
@@ -1225,13 +1226,13 @@ __global__ __launch_bounds__(128) void k_assemble_lines(AsmArgs A)
 {
 	if (!emitGo<EMIT>(A, true))   /* the counted totals do not fit, or nothing to emit */
 		return;
-	const uint32_t d = A.nDraws > 1 ? drawOfBlock(A.draws, A.nDraws, blockIdx.x) : 0u;
-	const AsmDraw& W = A.draws[d];
+	const uint32_t d = A.nDraws > 1 ? drawOfBlock(srpConst(A.draws), A.nDraws, blockIdx.x) : 0u;
+	const AsmDraw& W = srpConst(A.draws)[d];
 	const uint32_t k = (blockIdx.x - W.firstBlock) * 128u + threadIdx.x;
 	if (k >= W.nIn)
 		return;
 	const uint32_t g = W.primBase + k;   /* slot of this input in the count arrays */
-	const SrpDrawParams* P = W.P;
+	const SrpDrawParams* P = srpConst(W.P);
 	uint64_t s[2];
 	lineStream(W.prim, W.start, k, W.count, s);
 	uint32_t slot[2];
@@ -1329,13 +1330,13 @@ __global__ __launch_bounds__(128) void k_assemble_points(AsmArgs A)
 {
 	if (!emitGo<EMIT>(A, true))   /* the counted totals do not fit, or nothing to emit */
 		return;
-	const uint32_t d = A.nDraws > 1 ? drawOfBlock(A.draws, A.nDraws, blockIdx.x) : 0u;
-	const AsmDraw& W = A.draws[d];
+	const uint32_t d = A.nDraws > 1 ? drawOfBlock(srpConst(A.draws), A.nDraws, blockIdx.x) : 0u;
+	const AsmDraw& W = srpConst(A.draws)[d];
 	const uint32_t k = (blockIdx.x - W.firstBlock) * 128u + threadIdx.x;
 	if (k >= W.nIn)
 		return;
 	const uint32_t g = W.primBase + k;   /* slot of this input in the count arrays */
-	const SrpDrawParams* P = W.P;
+	const SrpDrawParams* P = srpConst(W.P);
 	const uint32_t slot = slotOf(W, W.start + k);
 	if (!slotsValid(A, P, &slot, 1))
 	{

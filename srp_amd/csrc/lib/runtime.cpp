@@ -1215,10 +1215,10 @@ bool varyingLayout(const SRPVertexShader* V, SrpDrawParams& H)
 		for (size_t e = 0; e < vi.nItems && words; e++)
 		{
 			if (nWords >= SRP_MAX_WORDS) { words = false; break; }
-			uint8_t k = SRP_WORD_PROVOKING;
-			if (vi.type == SRP_FLOAT && vi.interpolationMode == SRP_INTERPOLATION_MODE_PERSPECTIVE) k = SRP_WORD_PERSPECTIVE;
-			else if (vi.type == SRP_FLOAT && vi.interpolationMode == SRP_INTERPOLATION_MODE_AFFINE) k = SRP_WORD_AFFINE;
-			H.wordKind[nWords++] = k;
+			const uint32_t bit = 1u << nWords++;
+			if (vi.type == SRP_FLOAT && vi.interpolationMode == SRP_INTERPOLATION_MODE_PERSPECTIVE) H.wordPerspective |= bit;
+			else if (vi.type == SRP_FLOAT && vi.interpolationMode == SRP_INTERPOLATION_MODE_AFFINE) H.wordAffine |= bit;
+			else H.wordProvoking |= bit;
 		}
 		off += (uint32_t) (es * vi.nItems);
 	}

@@ -171,8 +171,8 @@ __global__ __launch_bounds__(256) void k_train_pass(TrainArgs A)
 	static_assert(SRP_NN_HID * TP_W1_ROW <= SRP_NN_ENC * TP_ROW && 4 * SRP_NN_HID + 3 <= SRP_NN_ENC, "LDS phases fit");
 	const int lane = (int) (threadIdx.x & 63u), wave = (int) (threadIdx.x >> 6);
 	const int g = lane >> 4, c = lane & 15;
-	const SrpNnDevice* net = A.net;
-	const uint16_t* w1 = net->w1;
+	const SrpNnDevice* net = srpConst(A.net);
+	const uint16_t* w1 = srpGlobal(net->w1);
 	uint4 w1v[SRP_NN_HID * SRP_NN_ENC / 8 / 256];
 #pragma unroll
 	for (int i = 0; i < SRP_NN_HID * SRP_NN_ENC / 8 / 256; i++)
@@ -195,12 +195,13 @@ __global__ __launch_bounds__(256) void k_train_pass(TrainArgs A)
 #pragma unroll
 	for (int i = 0; i < 2; i++)
 	{
-		wv[i] = *reinterpret_cast<const uint4*>(net->w2f + 8 * (256 * i + tid));
-		wv[2 + i] = *reinterpret_cast<const uint4*>(net->w2b + 8 * (256 * i + tid));
+		wv[i] = *reinterpret_cast<const uint4*>(srpGlobal(net->w2f) + 8 * (256 * i + tid));
+		wv[2 + i] = *reinterpret_cast<const uint4*>(srpGlobal(net->w2b) + 8 * (256 * i + tid));
 	}
-	wv[4] = *reinterpret_cast<const uint4*>(net->w3b + 8 * tid);
-	wv[5] = *reinterpret_cast<const uint4*>(net->w3f + 8 * (tid & 127));
-	const float bv = tid < 64 ? net->b1[tid] : (tid < 128 ? net->b2[tid - 64] : (tid < 131 ? net->b3[tid - 128] : 0.0f));
+	wv[4] = *reinterpret_cast<const uint4*>(srpGlobal(net->w3b) + 8 * tid);
+	wv[5] = *reinterpret_cast<const uint4*>(srpGlobal(net->w3f) + 8 * (tid & 127));
+	const float bv = tid < 64 ? srpGlobal(net->b1)[tid]
+	                          : (tid < 128 ? srpGlobal(net->b2)[tid - 64] : (tid < 131 ? srpGlobal(net->b3)[tid - 128] : 0.0f));
 	const size_t ld = A.batch;
 #pragma unroll
 	for (int i = 0; i < SRP_NN_HID * SRP_NN_ENC / 8 / 256; i++)
