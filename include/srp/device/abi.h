@@ -11,7 +11,7 @@
 #include <stdint.h>
 #include "srp/context.h"
 
-#define SRP_ABI_VERSION 17u
+#define SRP_ABI_VERSION 18u
 #define SRP_MAX_VARYINGS 16
 #define SRP_MAX_WORDS 32          /* fast interpolation path: 4-byte words */
 #define SRP_MAX_VARYING_BYTES 256 /* general path: bytes per fragment */
@@ -55,7 +55,8 @@ typedef struct SrpState
 	uint32_t lateZ;                   /* fragment shader may overwrite depth */
 } SrpState;
 
-/* Triangle after clipping and setup (one per assembled primitive). */
+/* Triangle after clipping and setup (one per assembled primitive): six
+ * 16-byte words, which the rasteriser loads whole. */
 typedef struct SrpTri
 {
 	float l0[3];           /* barycentrics at the bbox's first pixel centre */
@@ -66,8 +67,11 @@ typedef struct SrpTri
 	float invW[3];
 	float zw[3];           /* ndc z * invW per vertex */
 	uint32_t vref[3];      /* varying slots after the winding fix */
-	uint32_t pad;
+	uint32_t pad[2];
 } SrpTri;
+#ifdef __cplusplus
+static_assert(sizeof(SrpTri) == 96, "six 16-byte words");
+#endif
 
 typedef struct SrpLine
 {

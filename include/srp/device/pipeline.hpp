@@ -164,9 +164,9 @@ __device__ __forceinline__ uint32_t elemSize(uint32_t type)
  * ((A*invW)*w summed, times 1/sum(invW*w)), affine (A*w summed) or a copy
  * from the provoking vertex.  `out` stays in registers when the shader's
  * reads have constant offsets. */
-template <int N>
-__device__ __forceinline__ void interpWords(const SrpDrawParams* P, const uint32_t* const* v, const float* w,
-                                            const float* invW, float rec, uint32_t pv, uint32_t* out)
+template <int N, int MAX = SRP_MAX_WORDS, class Load4>
+__device__ __forceinline__ void interpWordsFrom(const SrpDrawParams* P, Load4&& load4, const float* w, const float* invW,
+                                                float rec, uint32_t pv, uint32_t* out)
 {
 	const uint32_t nWords = P->nWords;
 	const uint32_t persp = P->wordPerspective, affine = P->wordAffine, copied = P->wordProvoking;
@@ -176,7 +176,7 @@ __device__ __forceinline__ void interpWords(const SrpDrawParams* P, const uint32
 #pragma unroll
 	for (int k0 = 0; k0 < SRP_MAX_WORDS; k0 += 4)
 	{
-		if (k0 >= (int) nWords)
+		if (k0 >= MAX || k0 >= (int) nWords)
 		{
 #pragma unroll
 			for (int q = 0; q < 4; q++)
@@ -186,7 +186,7 @@ __device__ __forceinline__ void interpWords(const SrpDrawParams* P, const uint32
 		uint32_t a[N][4];
 #pragma unroll
 		for (int i = 0; i < N; i++)
-			__builtin_memcpy(a[i], v[i] + k0, 16);
+			load4(i, k0, a[i]);
 #pragma unroll
 		for (int q = 0; q < 4; q++)
 		{
@@ -212,6 +212,13 @@ __device__ __forceinline__ void interpWords(const SrpDrawParams* P, const uint32
 				out[k] = ((copied >> k) & 1u) ? (pv ? a[N - 1][q] : a[0][q]) : 0u;
 		}
 	}
+}
+
+template <int N>
+__device__ __forceinline__ void interpWords(const SrpDrawParams* P, const uint32_t* const* v, const float* w,
+                                            const float* invW, float rec, uint32_t pv, uint32_t* out)
+{
+	interpWordsFrom<N>(P, [&](int i, int k0, uint32_t* a) { __builtin_memcpy(a, v[i] + k0, 16); }, w, invW, rec, pv, out);
 }
 
 /* General path: any layout, byte addressed (interpolation.c:93-163). */
@@ -624,14 +631,16 @@ __global__ __launch_bounds__(256) void srp_raster_persistent16(SrpRasterLaunch L
 constexpr int RF = 128;
 
 /* Waves per SIMD the batched rasteriser kernels are compiled for (register
- * budget 512 / waves, so 72 VGPRs at 7).  Tiles are latency-bound and a
- * 1080p frame has a few thousand busy tiles, so the more of them resident
- * at once the better; 128-fragment batches keep LDS at 4.7 KB per wave.
- * Measured on the 1080p mesh: 5 waves 71.9 us, 6 71.6, 7 62.8, 8 70.1 (the
- * 64-register budget spills).  A wave-cooperative shader (a network on the
+ * budget 512 / waves, so 96 VGPRs at 5).  Tiles are latency-bound, so more
+ * of them resident at once help until the budget spills: 7 waves (72
+ * registers, up to 63 of them spilled) against 5 and 4 measured 1,918, 1,876
+ * and 1,850 us on 2,000 triangles at 512x512, 18.05, 17.71 and 18.41 ms on
+ * the 1080p mix, 1,214, 1,190 and 1,185 us on a scene of eight meshes, 7.25,
+ * 6.98 and 6.85 ms on a 20-scene batch.  128-fragment batches keep LDS at
+ * 4.7 KB per wave.  A wave-cooperative shader (a network on the
  * matrix cores) needs more than 128 registers and gets 2. */
 #ifndef SRP_RASTER_WAVES
-#define SRP_RASTER_WAVES 7
+#define SRP_RASTER_WAVES 5
 #endif
 
 /* Fragment shaders that evaluate a whole wave of fragments together (all 64
@@ -675,12 +684,44 @@ __device__ __forceinline__ bool monotoneOp(uint32_t op)
 }
 
 /* Barycentrics of tile pixel p (lane index layout) for triangle T. */
-__device__ __forceinline__ void baryAt(const SrpTri& T, int x, int y, float* l)
+template <class Tri>
+__device__ __forceinline__ void baryAt(const Tri& T, int x, int y, float* l)
 {
 	const int ny = y - (int) T.y0, nx = x - (int) T.x0;
 #pragma unroll
 	for (int e = 0; e < 3; e++)
 		l[e] = replay(replay(T.l0[e], T.dy[e], ny), T.dx[e], nx);
+}
+
+/* A triangle record in registers, read as its six 16-byte words: field by
+ * field it is some twenty loads, and when the lanes of a wave want different
+ * records each of them occupies the address unit for up to 64 cycles. */
+struct TriRegs
+{
+	float l0[3], dx[3], dy[3];
+	int x0, y0;
+	uint32_t flags, id;
+	float invW[3], zw[3];
+	uint32_t vref[3];
+};
+__device__ __forceinline__ TriRegs loadTri(const SrpTri* p)
+{
+	static_assert(offsetof(SrpTri, x0) == 36 && offsetof(SrpTri, flags) == 44 && offsetof(SrpTri, invW) == 52 &&
+	              offsetof(SrpTri, zw) == 64 && offsetof(SrpTri, vref) == 76, "word positions below");
+	const uint4* w = reinterpret_cast<const uint4*>(p);
+	const uint4 a = w[0], b = w[1], c = w[2], d = w[3], e = w[4], f = w[5];
+	auto F = [](uint32_t x) { return __uint_as_float(x); };
+	TriRegs T;
+	T.l0[0] = F(a.x); T.l0[1] = F(a.y); T.l0[2] = F(a.z);
+	T.dx[0] = F(a.w); T.dx[1] = F(b.x); T.dx[2] = F(b.y);
+	T.dy[0] = F(b.z); T.dy[1] = F(b.w); T.dy[2] = F(c.x);
+	T.x0 = (int) (c.y & 0xFFFFu); T.y0 = (int) (c.y >> 16);
+	T.flags = c.w;
+	T.id = d.x;
+	T.invW[0] = F(d.y); T.invW[1] = F(d.z); T.invW[2] = F(d.w);
+	T.zw[0] = F(e.x); T.zw[1] = F(e.y); T.zw[2] = F(e.z);
+	T.vref[0] = e.w; T.vref[1] = f.x; T.vref[2] = f.y;
+	return T;
 }
 
 /* Row bases of up to 8 triangles of a tile (the set bits of `round`, in
@@ -706,6 +747,50 @@ __device__ __forceinline__ void rowBases(const SrpTri* tris, const uint32_t* rec
 #pragma unroll
 	for (int e = 0; e < 3; e++)
 		base[j][i][e] = replay(replay(T.l0[e], T.dy[e], y - (int) T.y0), T.dx[e], cs - (int) T.x0);
+}
+
+/* A run's triangles (at most 8) while they are shaded pixel-parallel: their
+ * records and, when they have at most RUN_WORDS words, their vertices'
+ * varyings, copied to LDS together.  Read from memory one triangle after
+ * another, each pays the latency of its record and then of its varyings. */
+constexpr uint32_t RUN_WORDS = 8;
+struct RunStage
+{
+	SrpTri tri[8];
+	uint32_t words[8][3][RUN_WORDS];
+};
+
+/* rowBases for the first nk staged triangles.  Lanes 0..23 walk one
+ * (triangle, edge) each down to the tile's first row inside the box; lane
+ * (j, i) takes triangle j's three values on to row i (at most 7 additions,
+ * the same sequence) and then along the row. */
+__device__ __forceinline__ void runBases(const SrpTri* tris, uint32_t nk, uint32_t tx, uint32_t ty, uint32_t lane,
+                                         float (*base)[8][3])
+{
+	const uint32_t j = lane & 7u, i = lane >> 3;
+	const bool has = j < nk;
+	const SrpTri& T = tris[has ? j : 0u];
+	const int ys = ((int) (ty * 8u) > (int) T.y0) ? (int) (ty * 8u) : (int) T.y0;
+	float down = 0.0f;
+	if (has && i < 3u)
+		down = replay(T.l0[i], T.dy[i], ys - (int) T.y0);
+	const int y = (int) (ty * 8u + i);
+	const int n = y - ys;
+	float v[3];
+#pragma unroll
+	for (int e = 0; e < 3; e++)
+		v[e] = __shfl(down, (int) (j + 8u * (uint32_t) e));
+	if (!has || y < (int) T.y0 || y >= (int) T.y1)
+		return;
+#pragma unroll
+	for (int k = 0; k < 7; k++)
+#pragma unroll
+		for (int e = 0; e < 3; e++)
+			v[e] = k < n ? v[e] + T.dy[e] : v[e];
+	const int cs = ((int) (tx * 8u) > (int) T.x0) ? (int) (tx * 8u) : (int) T.x0;
+#pragma unroll
+	for (int e = 0; e < 3; e++)
+		base[j][i][e] = replay(v[e], T.dx[e], cs - (int) T.x0);
 }
 
 /* Barycentrics of pixel (px, py) inside triangle slot j's box from its row base. */
@@ -749,7 +834,14 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 	__shared__ float base[8][8][3];
 	__shared__ unsigned long long triMask[64];
 	__shared__ uint32_t fragBase[64];
-	__shared__ float fragL[3][RF];
+	/* barycentrics of listed fragments; or the triangles of a run */
+	__shared__ union
+	{
+		float fragL[3][RF];
+		RunStage run;
+	} sh;
+	static_assert(sizeof(RunStage) <= sizeof(float) * 3 * RF, "a run is staged where a list keeps barycentrics");
+	float (*fragL)[RF] = sh.fragL;
 	__shared__ uint8_t fragPix[RF];
 	__shared__ uint8_t fragTri[RF];
 	__shared__ uint32_t fragCol[RF];
@@ -853,24 +945,32 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 		const bool known = __shfl((int) sknown, (int) src) != 0;
 		uint32_t nb;
 		const uint64_t unkWin = __ballot(lane < avail && !known);
-		if (L.bigPixel && (unkWin & 1ull))
+		/* Which entries come next, and how.  A run shades up to 8 triangles
+		 * pixel-parallel: lane = pixel, the triangles in order, each fragment
+		 * tested and shaded as the reference does, with no fragment list; it
+		 * is meant for triangles without exact masks, which cover much of the
+		 * tile.  Those whose every fragment here must fail the depth test are
+		 * dropped first (srpTileDepthCull).  When any of the first 8 entries
+		 * that remain has no mask, a run takes them up to the last such one,
+		 * and the triangles with masks between them along (their coverage is
+		 * found again, the same): a tile whose list alternates between the
+		 * two kinds would otherwise pay a pass of one or two triangles for
+		 * every change (a 20-scene batch 6.98 -> 5.71 ms; requiring 2 or 3
+		 * of the 8 gave 5.74 and 5.85).  The list path takes the entries
+		 * before the first that has no mask. */
+		uint64_t keepRun = 0;    /* entries the run shades */
+		uint64_t dropped = 0;    /* entries without masks that cannot have a visible fragment */
+		uint32_t run = 0;        /* entries the run consumes; 0: the list path */
+		if (L.bigPixel && unkWin)
 		{
-			/* A run of triangles without exact masks heads the window:
-			 * lane = pixel, the triangles in order, each fragment tested
-			 * and shaded as the reference does, with no fragment list
-			 * (these triangles cover much of the tile).  Triangles whose
-			 * every fragment here must fail the depth test are dropped
-			 * first (srpTileDepthCull); the run then takes window entries
-			 * until it holds 8 triangles that remain. */
-			const uint64_t notUnk = ~unkWin;
-			const uint32_t runMax = notUnk ? (uint32_t) __builtin_ctzll(notUnk) : 64u;
-			uint64_t keep = (runMax >= 64u) ? ~0ull : ((1ull << runMax) - 1ull);
+			/* (a masked entry of no coverage has no record) */
+			uint64_t keep = unkWin | __ballot(lane < avail && mask != 0ull);
 			if (cull)
 			{
 				/* the tile's stored depth range (pixels inside the
-				 * framebuffer); a run's culls use its value at the run's
-				 * start, which is conservative because a monotone compare
-				 * only writes depths that make later fragments fail more */
+				 * framebuffer); the culls use its value here, which is
+				 * conservative because a monotone compare only writes
+				 * depths that make later fragments fail more */
 				float zMax = inFb ? dep : -__builtin_inff();
 				float zMin = inFb ? dep : __builtin_inff();
 				for (int off = 32; off > 0; off >>= 1)
@@ -879,29 +979,50 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 					zMin = fminf(zMin, __shfl_xor(zMin, off));
 				}
 				bool drop = false;
-				if (lane < runMax)
+				if ((unkWin >> lane) & 1ull)
 					drop = srpTileDepthCull(&L.tris[recIdx[(head + lane) & 63u]], tx, ty, st.depthOp, zMin, zMax);
-				keep &= ~__ballot(drop);
+				dropped = __ballot(drop);
+				keep &= ~dropped;
 			}
-			uint32_t run = runMax;
+			const uint64_t first = __ballot(((keep >> lane) & 1ull) && (uint32_t) __popcll(keep & ltMask) < 8u);
+			const uint64_t firstUnk = first & unkWin;
+			if (firstUnk)
 			{
-				uint64_t k = keep;
-				for (int c = 0; c < 8 && k; c++)
-					k &= k - 1ull;
-				if (k)
-					run = (uint32_t) __builtin_ctzll(k);   /* the 9th remaining entry starts the next run */
+				keepRun = first & (~0ull >> __builtin_clzll(firstUnk));
+				const uint64_t rest = keep & ~keepRun;
+				run = rest ? (uint32_t) __builtin_ctzll(rest) : avail;   /* dropped entries go with it */
 			}
-			const uint64_t keepRun = keep & ((run >= 64u) ? ~0ull : ((1ull << run) - 1ull));
-			if (keepRun)
+		}
+		if (run)
+		{
+			const uint32_t nk = (uint32_t) __popcll(keepRun);
+			const bool words = WORDS && !DEFER && P->nWords <= RUN_WORDS;   /* varyings staged too */
+			uint32_t* runRec = fragBase;   /* records of the kept triangles, in order */
+			if ((keepRun >> lane) & 1ull)
+				runRec[__popcll(keepRun & ltMask)] = recIdx[(head + lane) & 63u];
+			__syncthreads();
+			/* six 16-byte pieces a record */
+			const uint32_t sj = lane / 6u, sp = lane - 6u * sj;
+			if (sj < nk)
+				reinterpret_cast<uint4*>(&sh.run.tri[sj])[sp] = reinterpret_cast<const uint4*>(&L.tris[runRec[sj]])[sp];
+			__syncthreads();
+			/* lane (j, q): word q of triangle j's vertices, in flight while the bases are walked */
+			const uint32_t vj = lane >> 3, vq = lane & 7u;
+			const bool has = words && vj < nk && vq < P->nWords;
+			uint32_t vw[3] = {0u, 0u, 0u};
+			if (has)
+#pragma unroll
+				for (int k = 0; k < 3; k++)
+					vw[k] = reinterpret_cast<const uint32_t*>(varyingPtr(P, sh.run.tri[vj].vref[k]))[vq];
+			runBases(sh.run.tri, nk, tx, ty, lane, base);
+			if (has)
+#pragma unroll
+				for (int k = 0; k < 3; k++)
+					sh.run.words[vj][k][vq] = vw[k];
+			__syncthreads();
+			for (uint32_t jb = 0; jb < nk; jb++)
 			{
-				rowBases(L.tris, recIdx, head, keepRun, tx, ty, lane, base);
-				__syncthreads();
-			}
-			uint32_t jb = 0;   /* row-base slot: rank of the triangle among those kept */
-			for (uint64_t rest = keepRun; rest; rest &= rest - 1ull, jb++)
-			{
-				const uint32_t j = (uint32_t) __builtin_ctzll(rest);
-				const SrpTri& T = L.tris[recIdx[(head + j) & 63u]];
+				const SrpTri& T = sh.run.tri[jb];
 				bool cov = px >= (int) T.x0 && px < (int) T.x1 && py >= (int) T.y0 && py < (int) T.y1;
 				float l[3] = {0.0f, 0.0f, 0.0f};
 				if (cov)
@@ -909,7 +1030,9 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 					baryFromBase(T, base, jb, px, py, tx, l);
 					cov = insideTri(T, l);
 				}
-				const bool front = (T.flags >> 3) & 1u;
+				if (__ballot(cov) == 0ull)
+					continue;
+				const bool front = (__builtin_amdgcn_readfirstlane((int) T.flags) >> 3) & 1;
 				const FaceState sf = front ? face0 : face1;
 				const float iw[3] = {T.invW[0], T.invW[1], T.invW[2]};
 				float depth = 0.0f, rec = 0.0f;
@@ -938,6 +1061,8 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 						active = false;
 					}
 				}
+				if (__ballot(active) == 0ull)
+					continue;   /* nothing to shade */
 				SRPFragmentShaderIn in;
 				SRPFragmentShaderOut out;
 				out.color[0] = 0.0f; out.color[1] = 0.0f; out.color[2] = 0.0f; out.color[3] = 0.0f;
@@ -954,7 +1079,11 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 				in.primitiveID = T.id;
 				if (active && !DEFER)
 				{
-					if (WORDS)
+					if (WORDS && words)
+						interpWordsFrom<3, (int) RUN_WORDS>(P, [&](int k, int k0, uint32_t* a) {
+							__builtin_memcpy(a, &sh.run.words[jb][k][k0 & 4], 16);
+						}, l, iw, rec, pv, reinterpret_cast<uint32_t*>(buf));
+					else if (WORDS)
 					{
 						const uint32_t* v[3];
 #pragma unroll
@@ -999,7 +1128,7 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 					if (ok)
 					{
 						if (st.stencilEnabled) sten = stencilApply(sf.passOp, sten, sf);
-						col = DEFER ? recIdx[(head + j) & 63u] : packColor(out.color);
+						col = DEFER ? fragBase[jb] : packColor(out.color);
 						wrote = true;
 						if (st.depthTest && st.depthWrite)
 							dep = d;
@@ -1012,7 +1141,8 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 		else
 		{
 		/* entries taken by the fragment-list path this time */
-		const uint32_t lim = (L.bigPixel && unkWin) ? (uint32_t) __builtin_ctzll(unkWin) : avail;
+		const uint64_t stop = L.bigPixel ? unkWin & ~dropped : 0ull;
+		const uint32_t lim = stop ? (uint32_t) __builtin_ctzll(stop) : avail;
 		/* Inclusive scan of fragment counts; keep the longest prefix that fits. */
 		const uint32_t cnt = (lane < lim) ? (uint32_t) __popcll(mask) : 0u;
 		uint32_t incl = cnt;
@@ -1045,7 +1175,7 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 			}
 		}
 		/* ...other triangles pixel-parallel, storing their barycentrics. */
-		uint64_t unk = __ballot(lane < nb && !known);
+		uint64_t unk = __ballot(lane < nb && !known && mask != 0ull);
 		while (unk)
 		{
 			const uint64_t round = takeRound(unk);
@@ -1096,7 +1226,7 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 			{
 				const uint32_t b = fragTri[f];
 				fragRec = recIdx[(head + b) & 63u];
-				const SrpTri& T = L.tris[fragRec];
+				const TriRegs T = loadTri(&L.tris[fragRec]);
 				facing = ((T.flags >> 3) & 1u) ? FRAG_FRONT : 0;
 				const int fx = (int) (tx * 8 + (p & 7u)), fy = (int) (ty * 8 + (p >> 3));
 				float l[3];
@@ -1291,7 +1421,7 @@ __global__ __launch_bounds__(256) void srp_defer_gather(SrpRasterLaunch L)
 			continue;
 		const uint32_t k = off + r;
 		const uint32_t pix = L.deferList[2u * s];
-		const SrpTri& T = L.tris[L.deferList[2u * s + 1u]];
+		const TriRegs T = loadTri(&L.tris[L.deferList[2u * s + 1u]]);
 		const int px = (int) (pix % width), py = (int) (pix / width);
 		float l[3];
 		baryAt(T, px, py, l);

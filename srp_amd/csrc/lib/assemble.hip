@@ -245,7 +245,7 @@ __device__ bool setupTriangle(const SrpDrawParams* P, Vtx v0, Vtx v1, Vtx v2, ui
 		T.zw[i] = v[i].c[2] * v[i].invW;
 		T.vref[i] = v[i].vref;
 	}
-	T.pad = 0;
+	T.pad[0] = T.pad[1] = 0;
 	return true;
 }
 

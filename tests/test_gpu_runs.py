@@ -1,0 +1,62 @@
+"""The batched rasteriser's pixel-parallel runs on lists that alternate
+between triangles with and without exact masks, and with varyings below, at
+and above the words a run stages: every frame equals the one-lane-per-pixel
+rasteriser's, bit for bit."""
+import ctypes as C
+import importlib.util
+import os
+
+import numpy as np
+import pytest
+
+from scene_runner import REPO
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def cases():
+    spec = importlib.util.spec_from_file_location("perf_cases", os.path.join(REPO, "perf", "cases.py"))
+    m = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(m)
+    return m
+
+
+def triangles(n, size, seed):
+    """n clip-space triangles, every third small (masked when binned), the
+    others `size` wide, in random depth order."""
+    rng = np.random.default_rng(seed)
+    half = np.where(np.arange(n) % 3 == 0, 0.03, size)[:, None, None]
+    xy = rng.uniform(-1, 1, (n, 1, 2)) + half * rng.uniform(-1, 1, (n, 3, 2))
+    v = np.concatenate([xy, rng.uniform(-0.9, 0.9, (n, 3, 1)), rng.random((n, 3, 3))], -1)
+    return np.ascontiguousarray(v.reshape(-1, 6), np.float32)
+
+
+@pytest.mark.parametrize("words", [3, 8, 9, 12])
+@pytest.mark.parametrize("n,size,w,h", [(1, 0.9, 40, 24), (9, 0.5, 64, 64), (400, 0.25, 333, 211)])
+def test_mixed_lists_equal_the_lane_per_pixel_rasteriser(cases, words, n, size, w, h):
+    a = cases.api()
+    lib = C.CDLL(os.path.join(REPO, "srp_amd", "libsrp_amd.so"))
+    a.NewContext(a.context)
+    a.DepthTest(True)
+    a.DepthCompareOp(cases.CMP_LESS)
+    s = cases.State("test")
+    v = triangles(n, size, 11 * n + words)
+    vb = s.vertices(v, 24)
+    # the shader writes three words; the others are declared and never read
+    extra = [(words - 3, cases.T_FLOAT, cases.FLAT)] if words > 3 else []
+    p = a.program("sc_vsColorPass", [(3, cases.T_FLOAT, cases.PERSPECTIVE)] + extra, "sc_fsColor")
+    fb = s.framebuffer(w, h)
+    frames = []
+    try:
+        for batched in (0, 1):
+            lib.srpHipSetRasterOptions(batched, 1, 24)
+            cases.start_frame(a, fb)
+            a.DrawVertexBuffer(vb, fb, C.byref(p), cases.PRIM_TRIANGLES, 0, 3 * n)
+            a.FramebufferDownload(fb)
+            frames.append([x.copy() for x in s.images])
+    finally:
+        lib.srpHipSetRasterOptions(1, 1, 24)
+    assert np.count_nonzero(frames[0][0])
+    for x, y in zip(*frames):
+        assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
