@@ -26,7 +26,7 @@ def triangles(n, size, seed):
     """n clip-space triangles, every third small (masked when binned), the
     others `size` wide, in random depth order."""
     rng = np.random.default_rng(seed)
-    half = np.where(np.arange(n) % 3 == 0, 0.03, size)[:, None, None]
+    half = np.where(np.arange(n) % 3 == 2, 0.03, size)[:, None, None]
     xy = rng.uniform(-1, 1, (n, 1, 2)) + half * rng.uniform(-1, 1, (n, 3, 2))
     v = np.concatenate([xy, rng.uniform(-0.9, 0.9, (n, 3, 1)), rng.random((n, 3, 3))], -1)
     return np.ascontiguousarray(v.reshape(-1, 6), np.float32)
