@@ -24,10 +24,11 @@ def cases():
 
 def triangles(n, size, seed):
     """n clip-space triangles, every third small (masked when binned), the
-    others `size` wide, in random depth order."""
+    others `size` wide, in random depth order; the first spans the view."""
     rng = np.random.default_rng(seed)
     half = np.where(np.arange(n) % 3 == 2, 0.03, size)[:, None, None]
     xy = rng.uniform(-1, 1, (n, 1, 2)) + half * rng.uniform(-1, 1, (n, 3, 2))
+    xy[0] = [[-0.8, -0.8], [0.8, -0.7], [0.1, 0.9]]
     v = np.concatenate([xy, rng.uniform(-0.9, 0.9, (n, 3, 1)), rng.random((n, 3, 3))], -1)
     return np.ascontiguousarray(v.reshape(-1, 6), np.float32)
 
