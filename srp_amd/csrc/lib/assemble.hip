@@ -629,10 +629,109 @@ __device__ __forceinline__ bool emitGo(const AsmArgs& A, bool leader)
 	return fits && any;
 }
 
+/* fanTriangle of a filled triangle by a group of ROW_GROUP lanes that all
+ * hold it, lane gl of the group taking row gl of each band of tiles: the box
+ * scan of binTriangle, whose rows depend on each other only through the row
+ * start (dy added once per row, in order).  Same records, pairs and order. */
+constexpr uint32_t ROW_GROUP = 8;
+template <bool EMIT>
+__device__ __forceinline__ void fillRows(const AsmArgs& A, const AsmDraw& W, uint32_t gl, const Vtx& a, const Vtx& b,
+                                         const Vtx& c, uint32_t recBase, uint32_t idBase, uint32_t itemBase,
+                                         uint32_t& nRec, uint32_t& nItems)
+{
+	const SrpDrawParams* P = srpConst(W.P);
+	SrpTri T;
+	if (!setupTriangle(P, a, b, c, recBase - idBase, T))
+		return;
+	nRec = 1;
+	const bool fits = recBase < A.recCap;
+	if (EMIT && gl == 0)
+	{
+		if (fits)
+			A.tris[recBase] = T;
+		else
+			atomicOr(A.error, 2u);
+	}
+	if (T.x1 <= T.x0 || T.y1 <= T.y0)
+		return;
+	const uint32_t sh = P->tileShift;
+	const uint32_t tx0 = T.x0 >> sh, tx1 = (T.x1 - 1u) >> sh;
+	const uint32_t ty0 = T.y0 >> sh, ty1 = (T.y1 - 1u) >> sh;
+	if (isSpan(P, T))
+	{
+		nItems = (tx1 - tx0 + 1u) * (ty1 - ty0 + 1u);
+		if (gl == 0)
+		{
+			if (EMIT)
+				appendSpan(A, P, T, W.tileBase, itemBase, fits ? recBase : 0xFFFFFFFFu);
+			else
+			{
+				const uint64_t act = __ballot(1);
+				if (__lane_id() == (uint32_t) __builtin_ctzll(act))
+					atomicAdd(A.spanCount, (uint32_t) __popcll(act));
+			}
+		}
+	}
+	else
+	{
+		/* exact masks: 8x8 tiles, at most four of them a band */
+		const uint32_t gshift = __lane_id() & ~(ROW_GROUP - 1u);
+		float row[3] = {T.l0[0], T.l0[1], T.l0[2]};
+		float thr[3];
+		srp::dev::edgeThresholds(T.flags, thr);
+		int at = T.y0;   /* the row `row` belongs to */
+		for (uint32_t ty = ty0; ty <= ty1; ty++)
+		{
+			const int y = (int) (8u * ty + gl);
+			uint32_t bits = 0;   /* covered pixels of the row from column 8 tx0 on */
+			if (y >= (int) T.y0 && y < (int) T.y1)
+			{
+				for (; at < y; at++)
+#pragma unroll
+					for (int e = 0; e < 3; e++) row[e] += T.dy[e];
+				float l[3] = {row[0], row[1], row[2]};
+				const int xEnd = (int) T.x1 - (int) (8u * tx0);
+				for (int x = (int) T.x0 - (int) (8u * tx0); x < xEnd; x++)
+				{
+					bits |= (srp::dev::insideEdges(l, thr) ? 1u : 0u) << x;
+#pragma unroll
+					for (int e = 0; e < 3; e++) l[e] += T.dx[e];
+				}
+			}
+			/* lane gl < 4 gathers tile tx0 + gl: a byte of every row */
+			uint64_t m = 0;
+#pragma unroll
+			for (int k = 0; k < (int) ROW_GROUP; k++)
+			{
+				const uint32_t r = (uint32_t) __shfl((int) bits, k, (int) ROW_GROUP);
+				m |= (uint64_t) ((r >> (8u * (gl & 3u))) & 255u) << (8 * k);
+			}
+			const bool hit = gl < 4u && m != 0ull;
+			const uint32_t hits = (uint32_t) (__ballot(hit) >> gshift) & 255u;
+			if (EMIT && hit)
+			{
+				const uint32_t o = itemBase + nItems + (uint32_t) __builtin_popcount(hits & ((1u << gl) - 1u));
+				if (o < A.itemCap)
+				{
+					A.pairKeys[o] = W.tileBase + ty * P->tilesX + tx0 + gl;
+					A.pairVals[o] = o;
+					A.pairRec[o] = fits ? (recBase | 0x80000000u) : 0xFFFFFFFFu;
+					A.pairMask[o] = fits ? m : 0ull;
+				}
+			}
+			nItems += (uint32_t) __builtin_popcount(hits);
+		}
+	}
+	if (EMIT && gl == 0 && (uint64_t) itemBase + nItems > A.itemCap)
+		atomicOr(A.error, 2u);
+}
+
 /* Triangle draws (all polygon modes): primitive_assembly.c:37-135.  The
  * common case — all three vertices inside the frustum, trivially accepted
- * by clipping.c:74-78 — stays in registers. */
-template <bool EMIT>
+ * by clipping.c:74-78 — stays in registers.  ROWS (single draws of filled
+ * triangles): ROW_GROUP lanes per input, for draws too small to fill the
+ * chip with a lane each (ROWS_MAX_INPUTS). */
+template <bool EMIT, bool ROWS>
 __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 {
 	if (!emitGo<EMIT>(A, true))   /* the counted totals do not fit, or nothing to emit */
@@ -642,7 +741,10 @@ __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 			A.zero[z] = 0u;
 	const uint32_t d = A.nDraws > 1 ? drawOfBlock(srpConst(A.draws), A.nDraws, blockIdx.x) : 0u;
 	const AsmDraw& W = srpConst(A.draws)[d];
-	const uint32_t k = (blockIdx.x - W.firstBlock) * 128u + threadIdx.x;
+	constexpr uint32_t LANES = ROWS ? ROW_GROUP : 1u;
+	const uint32_t gl = ROWS ? threadIdx.x % ROW_GROUP : 0u;
+	const bool first = gl == 0u;   /* the lane that writes the input's counts */
+	const uint32_t k = (blockIdx.x - W.firstBlock) * (128u / LANES) + threadIdx.x / LANES;
 	if (k >= W.nIn)
 		return;
 	const uint32_t g = W.primBase + k;   /* slot of this input in the count arrays */
@@ -656,7 +758,7 @@ __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 		slot[i] = slotOf(W, s[i]);
 	if (!slotsValid(A, P, slot, 3))
 	{
-		if (!EMIT)
+		if (!EMIT && first)
 		{
 			A.recOff[g] = 0;
 			A.genOff[g] = 0;
@@ -678,7 +780,7 @@ __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 	const bool clip = codeOr != 0 && codeAnd == 0;
 	if (!EMIT)
 	{
-		const uint64_t want = __ballot(clip);
+		const uint64_t want = __ballot(clip && first);
 		if (want)
 		{
 			const uint32_t lane = __lane_id();
@@ -687,7 +789,7 @@ __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 			if (lane == leader)
 				at = atomicAdd(A.clipCount, (uint32_t) __builtin_popcountll(want));
 			at = (uint32_t) __shfl((int) at, (int) leader);
-			if (clip)
+			if (clip && first)
 				A.clipList[at + (uint32_t) __builtin_popcountll(want & ((1ull << lane) - 1ull))] = g;
 		}
 	}
@@ -704,9 +806,12 @@ __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 	if (codeOr == 0)
 	{
 		for (int i = 0; i < 3; i++) v[i].invW = divide(v[i].c);
-		fanTriangle<EMIT, !EMIT>(A, W, v[0], v[1], v[2], recBase, idBase, itemBase, nRec, nItems, false);
+		if (ROWS)
+			fillRows<EMIT>(A, W, gl, v[0], v[1], v[2], recBase, idBase, itemBase, nRec, nItems);
+		else
+			fanTriangle<EMIT, !EMIT>(A, W, v[0], v[1], v[2], recBase, idBase, itemBase, nRec, nItems, false);
 	}
-	if (!EMIT)
+	if (!EMIT && first)
 	{
 		A.recOff[g] = nRec;
 		A.genOff[g] = 0;
@@ -1430,7 +1535,10 @@ void launchClipped(const AsmArgs& A, bool emit, hipStream_t s, uint32_t clipped,
 	{
 		const uint64_t want = ((uint64_t) clipHint + clipHint / 4u + 7u) / 8u;
 		clipBlocks = (uint32_t) (want < 256u ? 256u : (want > 2048u ? 2048u : want));
-		clipBlocks = clipBlocks < blocks ? clipBlocks : blocks;
+		/* (a group per triangle of a draw that clips much of its few
+		 * inputs: limited to the main grid, 2,000 triangles of which half
+		 * are clipped took eight rounds, 117 + 144 us; 52 + 36 with a group each) */
+		clipBlocks = (uint64_t) clipBlocks < 16ull * blocks ? clipBlocks : 16u * blocks;
 	}
 	if (!clipBlocks)
 		return;
@@ -1453,9 +1561,15 @@ void launchAssemble(const AsmArgs& A, int kind, bool emit, hipStream_t s, uint32
 			 * similar earlier draw, a quarter more), at least 256 blocks
 			 * (the empty grid of a draw that clips nothing still costs its
 			 * dispatch), and never more blocks than the draw's main
-			 * assembly grid. */
-			if (emit) hipLaunchKernelGGL(k_assemble_tris<true>, dim3(blocks), dim3(128), 0, s, A);
-			else hipLaunchKernelGGL(k_assemble_tris<false>, dim3(blocks), dim3(128), 0, s, A);
+			 * assembly grid (which has 128 inputs a block) can list. */
+			if (A.rows)
+			{
+				const uint32_t rb = (uint32_t) (((uint64_t) A.rows * ROW_GROUP + 127u) / 128u);
+				if (emit) hipLaunchKernelGGL((k_assemble_tris<true, true>), dim3(rb), dim3(128), 0, s, A);
+				else hipLaunchKernelGGL((k_assemble_tris<false, true>), dim3(rb), dim3(128), 0, s, A);
+			}
+			else if (emit) hipLaunchKernelGGL((k_assemble_tris<true, false>), dim3(blocks), dim3(128), 0, s, A);
+			else hipLaunchKernelGGL((k_assemble_tris<false, false>), dim3(blocks), dim3(128), 0, s, A);
 			launchClipped(A, emit, s, clipped, clipHint);
 			break;
 		}

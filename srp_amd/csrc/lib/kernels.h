@@ -108,7 +108,20 @@ struct AsmArgs
 	 * ranges the emitting half fills), saving a launch */
 	uint32_t* zero;
 	uint32_t zeroCount;
+	/* single draws of filled triangles with exact masks: nonzero (the inputs)
+	 * to assemble each triangle with a group of lanes (ROWS_MAX_INPUTS) */
+	uint32_t rows;
 };
+
+/* Most inputs of a draw whose triangles are assembled by eight lanes each: a
+ * lane per triangle leaves SIMDs without a wave and the time is the longest
+ * box scan of a lane.  Measured on one textured sphere, us a draw with a lane
+ * and with eight lanes a triangle, in a 1080p frame (boxes up to the largest
+ * masked) and in 640x360: 4,096 triangles 326 / 207 and 194 / 96; 16,384
+ * 261 / 158 and 113 / 75; 65,536 170 / 116 and 91 / 82; 131,044 156 / 127 but
+ * 91.7 / 95.8, where the boxes are two or three pixels and the setup that the
+ * eight lanes repeat costs more than the scan. */
+constexpr uint32_t ROWS_MAX_INPUTS = 65536;
 
 /* kind: 0 triangles, 1 lines, 2 points.  clipped: how many triangles the
  * counting pass listed for clipping, when the caller knows it (0 skips the

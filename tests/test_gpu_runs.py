@@ -61,3 +61,42 @@ def test_mixed_lists_equal_the_lane_per_pixel_rasteriser(cases, words, n, size, 
     assert np.count_nonzero(frames[0][0])
     for x, y in zip(*frames):
         assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
+def boxes(n, seed):
+    """n triangles with boxes from one pixel to just above the largest that
+    is masked, at every alignment to the 8x8 tiles of a 256x256 frame."""
+    rng = np.random.default_rng(seed)
+    k = np.arange(n)
+    x0, y0 = (k * 5) % 229 + 0.25, (k * 3) % 231 + 0.25
+    bw, bh = k % 26 + 0.4, (k // 26) % 26 + 0.4
+    px = np.stack([x0, x0 + bw, x0 + bw * rng.random(n)], -1)
+    py = np.stack([y0 + bh * rng.random(n), y0, y0 + bh], -1)
+    v = np.concatenate([(px / 128 - 1)[..., None], (1 - py / 128)[..., None], rng.uniform(-0.9, 0.9, (n, 3, 1)), rng.random((n, 3, 3))], -1)
+    return np.ascontiguousarray(v.reshape(-1, 6), np.float32)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 676, 65535, 65536, 65537])
+def test_lanes_per_triangle_do_not_change_the_frame(cases, n):
+    """The first draw of n triangles and the last n of a draw of more than
+    the limit of the row-parallel assembly give the same frame (the first
+    triangles of the larger draw lie outside the view)."""
+    a = cases.api()
+    a.NewContext(a.context)
+    a.DepthTest(True)
+    a.DepthCompareOp(cases.CMP_LESS)
+    s = cases.State("test")
+    v = boxes(n, n)
+    pad = max(0, 65600 - n)
+    far = np.tile(np.array([5, 5, 0, 0, 0, 0], np.float32), (3 * pad, 1))
+    p = a.program("sc_vsColorPass", [(3, cases.T_FLOAT, cases.PERSPECTIVE)], "sc_fsColor")
+    frames = []
+    for data in (v, np.ascontiguousarray(np.concatenate([far, v]))):
+        vb = s.vertices(data, 24)
+        fb = s.framebuffer(256, 256)
+        cases.start_frame(a, fb)
+        a.DrawVertexBuffer(vb, fb, C.byref(p), cases.PRIM_TRIANGLES, 0, len(data))
+        a.FramebufferDownload(fb)
+        frames.append([x.copy() for x in s.images])
+    for x, y in zip(*frames):
+        assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
