@@ -15,6 +15,7 @@
  * line setup and DDA raster/line.c:34-86, points raster/point.c:32-118,
  * NDC to screen core/framebuffer.c:48-55. */
 #include "kernels.h"
+#include "srp/device/span_rows.h"
 
 #pragma clang fp contract(off)
 
@@ -249,14 +250,27 @@ __device__ bool setupTriangle(const SrpDrawParams* P, Vtx v0, Vtx v1, Vtx v2, ui
 	return true;
 }
 
+/* The tiles of a span: about a third of its box's.  With every tile of the
+ * box listed (and a mask written for each) 2,000 triangles at 512x512 took
+ * 1.68 ms a frame and the 1080p mix 17.9 ms (151 M pairs); with these 0.54
+ * and 9.8.  Finding them costs a thread some 30 instructions a tile row. */
+template <class Tri>
+__device__ __forceinline__ uint32_t spanTiles(const SrpDrawParams* P, const Tri& T)
+{
+	SrpSpanScan S;
+	srpSpanScanInit(&S, T.l0, T.dx, T.dy, (int) T.x0, (int) T.y0, (int) T.x1, (int) T.y1);
+	return srpSpanTiles(&S, P->tileShift);
+}
+
 /* Tiles a triangle is binned to.  A triangle whose bounding box is at
  * most P->maskBox (<= SRP_SMALL_BBOX) pixels on each side is scanned here exactly as the
  * reference scans it (raster/triangle.c:78-110: rows from the box origin,
  * dldy per row, dldx per pixel), giving one 64-bit coverage mask per 8x8
  * tile; tiles it does not cover get no entry (an empty entry would cost the
  * rasteriser a window slot, and sliver fans such as a sphere's poles pile
- * hundreds of them onto a few tiles).  Larger triangles are binned to every
- * tile of their box and their coverage is found by the rasteriser.  Calls
+ * hundreds of them onto a few tiles).  Larger triangles are binned to the
+ * tiles of their box that their edges let them reach, and their coverage is
+ * found by the rasteriser.  Calls
  * emit(tileKey, mask, known) in row-major tile order.  The counting pass
  * (EMIT false) needs only which tiles are covered: once every tile of a
  * band has a pixel, the band's remaining rows are stepped but not scanned. */
@@ -323,8 +337,8 @@ __device__ __forceinline__ uint32_t binTriangle(const SrpDrawParams* P, const Sr
 		}
 		return n;
 	}
-	/* every tile of the box, without a mask: written by k_expand_spans */
-	return (tx1 - tx0 + 1u) * (ty1 - ty0 + 1u);
+	/* the tiles its rows can reach, without masks: written by k_expand_spans */
+	return spanTiles(P, T);
 }
 
 /* True when binTriangle gives T one unmasked entry per tile of its box
@@ -338,9 +352,9 @@ __device__ __forceinline__ bool isSpan(const SrpDrawParams* P, const SrpTri& T)
 }
 
 /* Reserve a span-list entry (one atomic per group of lanes calling
- * together) and fill it: the pairs of T's box tiles, items item.. in
- * row-major tile order, record `rec` (0xFFFFFFFF: none). */
-__device__ void appendSpan(const AsmArgs& A, const SrpDrawParams* P, const SrpTri& T, uint32_t tileBase, uint32_t item,
+ * together) and fill it: `count` pairs, items item.., record `rec`
+ * (0xFFFFFFFF: none). */
+__device__ void appendSpan(const AsmArgs& A, const SrpDrawParams* P, uint32_t tileBase, uint32_t item, uint32_t count,
                            uint32_t rec)
 {
 	const uint64_t act = __ballot(1);
@@ -355,16 +369,13 @@ __device__ void appendSpan(const AsmArgs& A, const SrpDrawParams* P, const SrpTr
 		atomicOr(A.error, 2u);
 		return;
 	}
-	const uint32_t sh = P->tileShift;
-	const uint32_t tx0 = T.x0 >> sh, tx1 = (T.x1 - 1u) >> sh;
-	const uint32_t ty0 = T.y0 >> sh, ty1 = (T.y1 - 1u) >> sh;
 	SrpSpan sp;
 	sp.item = item;
+	sp.count = count;
 	sp.rec = rec;
-	sp.keyBase = tileBase + ty0 * P->tilesX + tx0;
-	sp.stride = P->tilesX;
-	sp.nx = tx1 - tx0 + 1u;
-	sp.ny = ty1 - ty0 + 1u;
+	sp.tileBase = tileBase;
+	sp.tilesX = P->tilesX;
+	sp.shift = P->tileShift;
 	A.spans[at] = sp;
 }
 
@@ -544,7 +555,7 @@ __device__ __forceinline__ void fanTriangle(const AsmArgs& A, const AsmDraw& W, 
 			});
 			if (isSpan(P, T))
 			{
-				appendSpan(A, P, T, W.tileBase, o, fits ? r : 0xFFFFFFFFu);
+				appendSpan(A, P, W.tileBase, o, np, fits ? r : 0xFFFFFFFFu);
 				o += np;
 			}
 			if (o > A.itemCap)
@@ -659,11 +670,11 @@ __device__ __forceinline__ void fillRows(const AsmArgs& A, const AsmDraw& W, uin
 	const uint32_t ty0 = T.y0 >> sh, ty1 = (T.y1 - 1u) >> sh;
 	if (isSpan(P, T))
 	{
-		nItems = (tx1 - tx0 + 1u) * (ty1 - ty0 + 1u);
+		nItems = spanTiles(P, T);
 		if (gl == 0)
 		{
 			if (EMIT)
-				appendSpan(A, P, T, W.tileBase, itemBase, fits ? recBase : 0xFFFFFFFFu);
+				appendSpan(A, P, W.tileBase, itemBase, nItems, fits ? recBase : 0xFFFFFFFFu);
 			else
 			{
 				const uint64_t act = __ballot(1);
@@ -937,7 +948,11 @@ __device__ __forceinline__ void clipFillFans(const AsmArgs& A, const AsmDraw& W,
 			const uint32_t tx0 = (uint32_t) x0 >> sh, ty0 = (uint32_t) y0 >> sh;
 			const uint32_t ntx = (((uint32_t) x1 - 1u) >> sh) - tx0 + 1u;
 			if (oSpan)
-				weight = ntx * ((((uint32_t) y1 - 1u) >> sh) - ty0 + 1u);
+			{
+				SrpSpanScan S;
+				srpSpanScanInit(&S, l0, dx, dy, x0, y0, x1, y1);
+				weight = srpSpanTiles(&S, sh);
+			}
 			else
 			{
 				/* exact masks: tileShift 3 */
@@ -987,10 +1002,7 @@ __device__ __forceinline__ void clipFillFans(const AsmArgs& A, const AsmDraw& W,
 			const unsigned long long at = (unsigned long long) itemBase + pairs + (wIncl - weight);
 			if (oSpan)
 			{
-				SrpTri S = {};
-				S.x0 = (uint16_t) x0; S.y0 = (uint16_t) y0;
-				S.x1 = (uint16_t) x1; S.y1 = (uint16_t) y1;
-				appendSpan(A, P, S, W.tileBase, (uint32_t) at, oFits ? oRec : 0xFFFFFFFFu);
+				appendSpan(A, P, W.tileBase, (uint32_t) at, weight, oFits ? oRec : 0xFFFFFFFFu);
 			}
 			else if (at < A.itemCap)
 			{
@@ -1482,34 +1494,79 @@ __global__ __launch_bounds__(128) void k_assemble_points(AsmArgs A)
 }
 
 /* The tile pairs of the spans listed by the emitting pass: one wave per
- * span at a time, lanes over its tiles (consecutive items, so the writes
- * coalesce).  The pairs equal what a per-tile loop in the emitting thread
- * would write: item item + k is tile (k % nx, k / nx) of the box. */
-__global__ __launch_bounds__(256) void k_expand_spans(const SrpSpan* spans, const uint32_t* count, uint32_t cap,
-                                                      uint32_t* pairKeys, uint32_t* pairVals, uint32_t* pairRec,
-                                                      unsigned long long* pairMask, uint32_t itemCap)
+ * span at a time.  Lane r finds the tiles of tile row r (64 rows a round),
+ * then the lanes take the listed tiles in order, each finding its row by
+ * bisection over the rows' running counts, so that consecutive items are
+ * written together.  (Pairs without masks: pairMask is only read for a pair
+ * marked exact, or one without a record, whose mask is zero.) */
+__global__ __launch_bounds__(256) void k_expand_spans(const SrpSpan* spans, const SrpTri* tris, const uint32_t* count,
+                                                      uint32_t cap, uint32_t* pairKeys, uint32_t* pairVals,
+                                                      uint32_t* pairRec, unsigned long long* pairMask, uint32_t itemCap)
 {
 	const uint32_t lane = threadIdx.x & 63u;
-	const uint32_t wave = blockIdx.x * 4u + (threadIdx.x >> 6);
+	const uint32_t wave = (uint32_t) __builtin_amdgcn_readfirstlane((int) (blockIdx.x * 4u + (threadIdx.x >> 6)));
 	const uint32_t nWaves = gridDim.x * 4u;
 	uint32_t n = *count;
 	if (n > cap)
 		n = cap;
+	spans = srpConst(spans);
+	tris = srpConst(tris);
 	for (uint32_t i = wave; i < n; i += nWaves)
 	{
 		const SrpSpan sp = spans[i];
-		const uint32_t total = sp.nx * sp.ny;
-		const uint64_t m = (sp.rec == 0xFFFFFFFFu) ? 0ull : ~0ull;
-		for (uint32_t k = lane; k < total; k += 64u)
+		if (sp.rec == 0xFFFFFFFFu)
 		{
-			const uint32_t o = sp.item + k;
-			if (o >= itemCap)
-				break;
-			const uint32_t dy = k / sp.nx, dx = k - dy * sp.nx;
-			pairKeys[o] = sp.keyBase + dy * sp.stride + dx;
-			pairVals[o] = o;
-			pairRec[o] = sp.rec;
-			pairMask[o] = m;
+			/* no record to find the tiles from: empty pairs of any tile */
+			for (uint32_t k = lane; k < sp.count; k += 64u)
+			{
+				const uint32_t o = sp.item + k;
+				if (o >= itemCap)
+					break;
+				pairKeys[o] = sp.tileBase;
+				pairVals[o] = o;
+				pairRec[o] = 0xFFFFFFFFu;
+				pairMask[o] = 0ull;
+			}
+			continue;
+		}
+		const SrpTri* T = tris + sp.rec;
+		SrpSpanScan S;
+		srpSpanScanInit(&S, T->l0, T->dx, T->dy, (int) T->x0, (int) T->y0, (int) T->x1, (int) T->y1);
+		const uint32_t ty0 = (uint32_t) T->y0 >> sp.shift, ny = (((uint32_t) T->y1 - 1u) >> sp.shift) - ty0 + 1u;
+		uint32_t item = sp.item;
+		for (uint32_t r0 = 0; r0 < ny; r0 += 64u)
+		{
+			uint32_t a = 0, b = 0, cnt = 0;
+			if (r0 + lane < ny && srpSpanRow(&S, ty0 + r0 + lane, sp.shift, &a, &b))
+				cnt = b - a + 1u;
+			uint32_t incl = cnt;
+#pragma unroll
+			for (uint32_t off = 1; off < 64; off <<= 1)
+			{
+				const uint32_t v = __shfl_up(incl, off);
+				if (lane >= off) incl += v;
+			}
+			const uint32_t total = __shfl(incl, 63);
+			const uint32_t firstKey = sp.tileBase + (ty0 + r0 + lane) * sp.tilesX + a - (incl - cnt);
+			for (uint32_t k0 = 0; k0 < total; k0 += 64u)
+			{
+				const uint32_t k = k0 + lane;
+				/* the first row whose running count passes k */
+				uint32_t row = 0;
+#pragma unroll
+				for (uint32_t step = 32; step > 0; step >>= 1)
+					if (__shfl(incl, (int) (row + step - 1u)) <= k)
+						row += step;
+				const uint32_t key = __shfl(firstKey, (int) (row & 63u)) + k;
+				const uint32_t o = item + k;
+				if (k < total && o < itemCap)
+				{
+					pairKeys[o] = key;
+					pairVals[o] = o;
+					pairRec[o] = sp.rec;
+				}
+			}
+			item += total;
 		}
 	}
 }
@@ -1517,8 +1574,8 @@ __global__ __launch_bounds__(256) void k_expand_spans(const SrpSpan* spans, cons
 void launchExpandSpans(const AsmArgs& A, uint32_t blocks, hipStream_t s)
 {
 	if (blocks)
-		hipLaunchKernelGGL(k_expand_spans, dim3(blocks), dim3(256), 0, s, A.spans, A.spanCount, A.spanCap, A.pairKeys,
-		                   A.pairVals, A.pairRec, A.pairMask, A.itemCap);
+		hipLaunchKernelGGL(k_expand_spans, dim3(blocks), dim3(256), 0, s, A.spans, A.tris, A.spanCount, A.spanCap,
+		                   A.pairKeys, A.pairVals, A.pairRec, A.pairMask, A.itemCap);
 }
 
 void launchClipped(const AsmArgs& A, bool emit, hipStream_t s, uint32_t clipped, uint32_t clipHint)

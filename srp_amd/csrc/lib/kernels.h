@@ -35,16 +35,17 @@ struct AsmDraw
 	uint32_t firstBlock;  /* first block of the draw in the launch */
 };
 
-/* A triangle binned to every tile of its box (no exact masks): its tile
- * pairs are items item .. item + nx*ny - 1, tile (dx, dy) of the box at
- * item + dy*nx + dx with key keyBase + dy*stride + dx (k_expand_spans). */
+/* A triangle binned without exact masks: its tile pairs are items item ..
+ * item + count - 1, the tiles that its rows list (srp/device/span_rows.h) in
+ * row-major order, written by k_expand_spans. */
 struct SrpSpan
 {
 	uint32_t item;
+	uint32_t count;
 	uint32_t rec;         /* triangle record, 0xFFFFFFFF: none (capacity exceeded) */
-	uint32_t keyBase;     /* tile key of the box's first tile */
-	uint32_t stride;      /* tiles per framebuffer row */
-	uint32_t nx, ny;      /* box size in tiles */
+	uint32_t tileBase;    /* first tile of the draw's framebuffer */
+	uint32_t tilesX;      /* tiles per framebuffer row */
+	uint32_t shift;       /* log2 of the tile side */
 };
 
 /* Arguments of the assembly kernels (assemble.hip). */
