@@ -615,17 +615,10 @@ __device__ __forceinline__ void fanTriangle(const AsmArgs& A, const AsmDraw& W, 
 	}
 }
 
-/* Start of an emitting kernel of a single draw (AsmArgs.fitTotals): false
- * when it has nothing to do, because the counted totals do not fit the
- * capacities it was given or nothing was assembled.  Block 0 of the
- * leading kernel records the outcome and publishes the counters. */
-template <bool EMIT>
-__device__ __forceinline__ bool emitGo(const AsmArgs& A, bool leader)
+/* emitGo below, for the totals t64 (records, generated vertices, items). */
+__device__ __forceinline__ bool fitGo(const AsmArgs& A, bool leader, const unsigned long long* t64)
 {
-	if (!EMIT || !A.fitTotals)
-		return true;
 	uint32_t* t = A.fitTotals;
-	const unsigned long long* t64 = reinterpret_cast<const unsigned long long*>(t + 8);
 	const FitCaps& c = A.fitCaps;
 	const bool fits = t64[0] <= c.records && t64[1] <= c.generated && t64[2] <= c.items &&
 	                  (unsigned long long) t[6] <= c.spans && (unsigned long long) t[4] <= c.clipped;
@@ -638,6 +631,18 @@ __device__ __forceinline__ bool emitGo(const AsmArgs& A, bool leader)
 			publish(t, A.fitHost, A.fitSeq);
 	}
 	return fits && any;
+}
+
+/* Start of an emitting kernel of a single draw (AsmArgs.fitTotals): false
+ * when it has nothing to do, because the counted totals do not fit the
+ * capacities it was given or nothing was assembled.  Block 0 of the
+ * leading kernel records the outcome and publishes the counters. */
+template <bool EMIT>
+__device__ __forceinline__ bool emitGo(const AsmArgs& A, bool leader)
+{
+	if (!EMIT || !A.fitTotals)
+		return true;
+	return fitGo(A, leader, reinterpret_cast<const unsigned long long*>(A.fitTotals + 8));
 }
 
 /* fanTriangle of a filled triangle by a group of ROW_GROUP lanes that all
@@ -737,6 +742,71 @@ __device__ __forceinline__ void fillRows(const AsmArgs& A, const AsmDraw& W, uin
 		atomicOr(A.error, 2u);
 }
 
+/* Emitting pass with ownScan: the counts before each group's input, from the
+ * counting pass's counts, and the fit check of their totals (block 0 stores
+ * them where the scan would).  False when there is nothing to emit. */
+__device__ __forceinline__ bool ownOffsets(const AsmArgs& A, uint32_t& rec, uint32_t& item)
+{
+	constexpr uint32_t PER = 128u / ROW_GROUP;   /* inputs of a block */
+	__shared__ unsigned long long tot[2][2];     /* [wave][records, items] */
+	__shared__ uint32_t bef[2][2];
+	__shared__ uint32_t own[2][PER];
+	const uint32_t n = A.rows, first = blockIdx.x * PER;
+	const uint32_t t = threadIdx.x, wave = t >> 6;
+	unsigned long long r64 = 0, i64 = 0;
+	uint32_t rb = 0, ib = 0;
+#pragma unroll 4
+	for (uint32_t i = t; i < n; i += 128u)
+	{
+		const uint32_t r = A.recOff[i], it = A.itemOff[i];
+		r64 += r;
+		i64 += it;
+		rb += i < first ? r : 0u;
+		ib += i < first ? it : 0u;
+		if (i >= first && i < first + PER)
+		{
+			own[0][i - first] = r;
+			own[1][i - first] = it;
+		}
+	}
+#pragma unroll
+	for (int off = 32; off > 0; off >>= 1)
+	{
+		r64 += __shfl_xor(r64, off);
+		i64 += __shfl_xor(i64, off);
+		rb += __shfl_xor(rb, off);
+		ib += __shfl_xor(ib, off);
+	}
+	if ((t & 63u) == 0u)
+	{
+		tot[wave][0] = r64;
+		tot[wave][1] = i64;
+		bef[wave][0] = rb;
+		bef[wave][1] = ib;
+	}
+	__syncthreads();
+	const unsigned long long totals[3] = {tot[0][0] + tot[1][0], 0ull, tot[0][1] + tot[1][1]};
+	if (blockIdx.x == 0 && t == 0)
+	{
+		unsigned long long* t64 = reinterpret_cast<unsigned long long*>(A.fitTotals + 8);
+		for (int k = 0; k < 3; k++)
+		{
+			t64[k] = totals[k];
+			A.fitTotals[k] = (uint32_t) totals[k];
+		}
+	}
+	if (!fitGo(A, true, totals))
+		return false;
+	rec = bef[0][0] + bef[1][0];
+	item = bef[0][1] + bef[1][1];
+	for (uint32_t k = 0; k < t / ROW_GROUP; k++)
+	{
+		rec += own[0][k];
+		item += own[1][k];
+	}
+	return true;
+}
+
 /* Triangle draws (all polygon modes): primitive_assembly.c:37-135.  The
  * common case — all three vertices inside the frustum, trivially accepted
  * by clipping.c:74-78 — stays in registers.  ROWS (single draws of filled
@@ -745,7 +815,13 @@ __device__ __forceinline__ void fillRows(const AsmArgs& A, const AsmDraw& W, uin
 template <bool EMIT, bool ROWS>
 __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 {
-	if (!emitGo<EMIT>(A, true))   /* the counted totals do not fit, or nothing to emit */
+	uint32_t ownRec = 0, ownItem = 0;   /* with ownScan: the counts before this input */
+	if (EMIT && ROWS && A.ownScan)
+	{
+		if (!ownOffsets(A, ownRec, ownItem))
+			return;
+	}
+	else if (!emitGo<EMIT>(A, true))   /* the counted totals do not fit, or nothing to emit */
 		return;
 	if (!EMIT && A.zero)
 		for (uint32_t z = blockIdx.x * 128u + threadIdx.x; z < A.zeroCount; z += gridDim.x * 128u)
@@ -807,7 +883,12 @@ __global__ __launch_bounds__(128) void k_assemble_tris(AsmArgs A)
 	if (clip)
 		return;
 	uint32_t recBase = 0, itemBase = 0, idBase = 0;
-	if (EMIT)
+	if (EMIT && ROWS && A.ownScan)
+	{
+		recBase = ownRec;
+		itemBase = ownItem;
+	}
+	else if (EMIT)
 	{
 		recBase = A.recOff[g];
 		itemBase = A.itemOff[g];

@@ -112,7 +112,18 @@ struct AsmArgs
 	/* single draws of filled triangles with exact masks: nonzero (the inputs)
 	 * to assemble each triangle with a group of lanes (ROWS_MAX_INPUTS) */
 	uint32_t rows;
+	/* emitting pass of such a draw, nothing clipped: recOff and itemOff hold
+	 * the counting pass's counts, not their scans; each block adds up those
+	 * before it (and all, for the fit check) itself */
+	uint32_t ownScan;
 };
+
+/* Most inputs of a draw whose emitting blocks add up the counts themselves:
+ * each reads them all (eight bytes an input), against two scan launches of
+ * 4.5 us each.  Frame with one such draw of a sphere at 320x180, us with the
+ * launches and their own scans: 576 triangles 83 and 79, 4,096 65 and 57,
+ * 8,100 71 and 71, 16,384 71 and 77. */
+constexpr uint32_t OWN_SCAN_MAX_INPUTS = 4096;
 
 /* Most inputs of a draw whose triangles are assembled by eight lanes each: a
  * lane per triangle leaves SIMDs without a wave and the time is the longest
@@ -160,6 +171,14 @@ void scanReserve(ScanScratch& scratch, size_t n, int nArrays);
  * n is a capacity and the count is min(n, *nDev), read on the device. */
 void tileBounds(const uint32_t* keys, size_t n, uint32_t* start, uint32_t* end, hipStream_t s,
                 const uint32_t* nDev = nullptr);
+
+/* Stable sort of the first min(cap, *nDev) items by tile (bits <= 16 bits of
+ * the keys, which fit them) in one launch: order[i] is the index of the item
+ * at place i; start and end of each tile that received one are set.  cap <=
+ * TS_MAX_ITEMS. */
+constexpr uint32_t TS_MAX_ITEMS = 16384;
+void tileSort(const uint32_t* keys, size_t cap, int bits, uint32_t* order, uint32_t* start, uint32_t* end, hipStream_t s,
+              const uint32_t* nDev);
 
 struct SortScratch
 {

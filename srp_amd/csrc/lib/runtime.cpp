@@ -1107,6 +1107,35 @@ void srp_lib_scan_exact(const uint32_t* counts, size_t n, int nArrays, uint32_t*
 	if (sc.buf64) HIP_CHECK(hipFree(sc.buf64));
 }
 
+/* Test hook (not part of the public headers): the one-launch sort by tile of
+ * small draws, on host data.  keys hold cap items below nTiles; the first
+ * count are sorted; order, start[nTiles] and end[nTiles] receive the result
+ * (tiles without items keep 0). */
+void srp_lib_tile_sort(const uint32_t* keys, size_t cap, size_t count, uint32_t nTiles, uint32_t* order, uint32_t* start,
+                       uint32_t* end)
+{
+	resolvePending();
+	int bits = 0;
+	while ((1ull << bits) < nTiles) bits++;
+	if (cap > TS_MAX_ITEMS || count > cap || bits > 16)
+		return;
+	Runtime& R = rt();
+	uint32_t* d = nullptr;
+	const size_t words = 2 * cap + 2 * (size_t) nTiles + 1;
+	HIP_CHECK(hipMalloc((void**) &d, words * sizeof(uint32_t) + 16));
+	uint32_t *dk = d, *dOrd = d + cap, *dRange = d + 2 * cap, *dn = dRange + 2 * (size_t) nTiles;
+	const uint32_t count32 = (uint32_t) count;
+	HIP_CHECK(hipMemcpyAsync(dk, keys, cap * sizeof(uint32_t), hipMemcpyHostToDevice, R.stream));
+	HIP_CHECK(hipMemcpyAsync(dn, &count32, sizeof(uint32_t), hipMemcpyHostToDevice, R.stream));
+	fillU32(dRange, 0u, 2 * (size_t) nTiles, R.stream);
+	tileSort(dk, cap, bits, dOrd, dRange, dRange + nTiles, R.stream, dn);
+	HIP_CHECK(hipMemcpyAsync(order, dOrd, count * sizeof(uint32_t), hipMemcpyDeviceToHost, R.stream));
+	HIP_CHECK(hipMemcpyAsync(start, dRange, nTiles * sizeof(uint32_t), hipMemcpyDeviceToHost, R.stream));
+	HIP_CHECK(hipMemcpyAsync(end, dRange + nTiles, nTiles * sizeof(uint32_t), hipMemcpyDeviceToHost, R.stream));
+	HIP_CHECK(hipStreamSynchronize(R.stream));
+	HIP_CHECK(hipFree(d));
+}
+
 /* Test hook (not part of the public headers): the stable radix sort the
  * draws use, on host data, with the runtime's own sort scratch.  keys and
  * vals hold cap items; the first count of them (count <= cap, read on the
@@ -1357,9 +1386,15 @@ void enqueueEmit(Runtime& R, const FitCaps& want, bool speculative)
 	{
 		/* spans: the grid strides over the device-side count */
 		launchExpandSpans(A, (uint32_t) std::min<unsigned long long>((caps.spans + 3) / 4, 2048ull), R.stream);
-		uint32_t *keys, *vals;
-		radixSort(A.pairKeys, A.pairVals, caps.items, bitsFor(D.nTiles), R.sort, &keys, &vals, R.stream, items);
-		tileBounds(keys, caps.items, tileStart, tileEnd, R.stream, items);
+		uint32_t *keys, *vals = A.pairVals;
+		const int tileBits = bitsFor(D.nTiles);
+		if (caps.items <= TS_MAX_ITEMS && tileBits <= 16)
+			tileSort(A.pairKeys, caps.items, tileBits, vals, tileStart, tileEnd, R.stream, items);
+		else
+		{
+			radixSort(A.pairKeys, A.pairVals, caps.items, tileBits, R.sort, &keys, &vals, R.stream, items);
+			tileBounds(keys, caps.items, tileStart, tileEnd, R.stream, items);
+		}
 		SrpRasterLaunch rl = D.rl;
 		rl.tris = A.tris;
 		rl.tileList = vals;
@@ -1423,7 +1458,11 @@ void enqueueCount(Runtime& R, bool clipSkipped)
 	A.zero = D.tileStart;
 	A.zeroCount = D.tileStart ? 2u * D.nTiles : 0u;
 	launchAssemble(A, D.kind, false, R.stream, clipSkipped ? 0u : kClipUnknown, D.clipHint);
-	scanExclusiveMulti(A.recOff, (size_t) D.nIn + 1, 3, D.nIn, totals, R.scan, R.stream,
+	/* a small draw's emitting blocks add up the counts themselves, unless it
+	 * clips: the clipped triangles' kernel needs the scans */
+	D.A.ownScan = (D.emitted && clipSkipped && A.rows && D.nIn <= OWN_SCAN_MAX_INPUTS) ? 1u : 0u;
+	if (!D.A.ownScan)
+		scanExclusiveMulti(A.recOff, (size_t) D.nIn + 1, 3, D.nIn, totals, R.scan, R.stream,
 	                   reinterpret_cast<unsigned long long*>(totals + 8));
 }
 

@@ -100,3 +100,30 @@ def test_lanes_per_triangle_do_not_change_the_frame(cases, n):
         frames.append([x.copy() for x in s.images])
     for x, y in zip(*frames):
         assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 1023, 1024, 1025, 4096, 4097])
+def test_repeated_small_draws_do_not_change_the_frame(cases, n):
+    """A draw seen before is enqueued whole, its emitting blocks adding up
+    the counts before theirs: the same frame as the first time, also after
+    the vertices moved (other counts, same number) and back."""
+    a = cases.api()
+    a.NewContext(a.context)
+    a.DepthTest(True)
+    a.DepthCompareOp(cases.CMP_LESS)
+    s = cases.State("test")
+    v = boxes(n, n)
+    moved = v.copy()
+    moved[:, 0] += np.float32(0.37)
+    p = a.program("sc_vsColorPass", [(3, cases.T_FLOAT, cases.PERSPECTIVE)], "sc_fsColor")
+    frames = {}
+    for name, data in (("v", v), ("m", moved)):
+        vb = s.vertices(data, 24)
+        fb = s.framebuffer(256, 256)
+        for turn in range(3):
+            cases.start_frame(a, fb)
+            a.DrawVertexBuffer(vb, fb, C.byref(p), cases.PRIM_TRIANGLES, 0, len(data))
+            a.FramebufferDownload(fb)
+            got = [x.copy() for x in s.images]
+            for x, y in zip(frames.setdefault(name, got), got):
+                assert np.array_equal(x.view(np.uint8), y.view(np.uint8))

@@ -62,3 +62,36 @@ def test_radix_sort_matches_stable_argsort():
         order = np.argsort(digit, kind="stable")
         assert np.array_equal(v[:count], vals[:count][order]), (cap, count, bits, kind)
         assert np.array_equal(k[:count], keys[:count][order]), (cap, count, bits, kind)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cap,count,tiles,kind", [
+    (1, 1, 1, "tiles"),             # no digit at all: one tile
+    (64, 0, 300, "tiles"),          # nothing counted
+    (64, 63, 2, "tiles"),
+    (1_025, 1_024, 255, "tiles"),   # one full round of the block, one digit
+    (5_000, 1_025, 257, "tiles"),   # a second round, two digits
+    (16_384, 16_383, 3_600, "same"),
+    (16_384, 16_384, 65_536, "uniform"),
+    (16_384, 16_384, 32_400, "tiles"),
+])
+def test_one_launch_tile_sort(cap, count, tiles, kind):
+    lib = ctypes.CDLL(LIB, mode=ctypes.RTLD_LOCAL)
+    lib.srp_lib_tile_sort.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_size_t, ctypes.c_uint32,
+                                      ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    rng = np.random.default_rng(21)
+    if kind == "same":
+        keys = np.full(cap, tiles - 1, np.uint32)
+    elif kind == "uniform":
+        keys = rng.integers(0, tiles, size=cap, dtype=np.uint32)
+    else:
+        keys = np.minimum(np.repeat(rng.integers(0, tiles, size=cap // 4 + 1), 4)[:cap] + np.arange(cap) % 3,
+                          tiles - 1).astype(np.uint32)
+    order, start, end = (np.full(max(n, 1), 7, np.uint32) for n in (cap, tiles, tiles))
+    lib.srp_lib_tile_sort(keys.ctypes.data, cap, count, tiles, order.ctypes.data, start.ctypes.data, end.ctypes.data)
+    want = np.argsort(keys[:count], kind="stable")
+    assert np.array_equal(order[:count], want)
+    first = np.searchsorted(keys[:count][want], np.arange(tiles), "left")
+    last = np.searchsorted(keys[:count][want], np.arange(tiles), "right")
+    some = last > first
+    assert np.array_equal(start, np.where(some, first, 0)) and np.array_equal(end, np.where(some, last, 0))
