@@ -302,6 +302,9 @@ struct FbImpl
 	uint32_t* dColor = nullptr;
 	float* dDepth = nullptr;
 	uint8_t* dStencil = nullptr;
+	uint32_t* hColor = nullptr;   /* the pinned host arrays as allocated */
+	float* hDepth = nullptr;
+	uint8_t* hStencil = nullptr;
 	bool deferred = false;
 	/* Deferred mode: clears and fills are recorded and run as one fused
 	 * kernel before the next use of the device copy. */
@@ -322,11 +325,25 @@ void fbFlushFills(FbImpl* F)
 	F->pendColor = F->pendDepth = F->pendStencil = false;
 }
 
+/* The public arrays are the pinned ones the framebuffer was made with (a
+ * caller may have put its own, pageable memory there): kernels can reach
+ * them. */
+bool fbOwnArrays(const FbImpl* F)
+{
+	return F->pub.color == F->hColor && F->pub.depth == F->hDepth && F->pub.stencil == F->hStencil;
+}
+
 void fbUpload(FbImpl* F)
 {
 	Runtime& R = rt();
 	F->pendColor = F->pendDepth = F->pendStencil = false;  /* the host arrays win */
 	const size_t n = F->pub.size;
+	if (fbOwnArrays(F))
+	{
+		copyArrays({{F->pub.color, F->pub.depth, F->pub.stencil}, {F->dColor, F->dDepth, F->dStencil}, {n * 4, n * 4, n}},
+		           R.stream);
+		return;
+	}
 	HIP_CHECK(hipMemcpyAsync(F->dColor, F->pub.color, n * 4, hipMemcpyHostToDevice, R.stream));
 	HIP_CHECK(hipMemcpyAsync(F->dDepth, F->pub.depth, n * 4, hipMemcpyHostToDevice, R.stream));
 	HIP_CHECK(hipMemcpyAsync(F->dStencil, F->pub.stencil, n, hipMemcpyHostToDevice, R.stream));
@@ -337,9 +354,15 @@ void fbDownload(FbImpl* F)
 	Runtime& R = rt();
 	fbFlushFills(F);
 	const size_t n = F->pub.size;
-	HIP_CHECK(hipMemcpyAsync(F->pub.color, F->dColor, n * 4, hipMemcpyDeviceToHost, R.stream));
-	HIP_CHECK(hipMemcpyAsync(F->pub.depth, F->dDepth, n * 4, hipMemcpyDeviceToHost, R.stream));
-	HIP_CHECK(hipMemcpyAsync(F->pub.stencil, F->dStencil, n, hipMemcpyDeviceToHost, R.stream));
+	if (fbOwnArrays(F))
+		copyArrays({{F->dColor, F->dDepth, F->dStencil}, {F->pub.color, F->pub.depth, F->pub.stencil}, {n * 4, n * 4, n}},
+		           R.stream);
+	else
+	{
+		HIP_CHECK(hipMemcpyAsync(F->pub.color, F->dColor, n * 4, hipMemcpyDeviceToHost, R.stream));
+		HIP_CHECK(hipMemcpyAsync(F->pub.depth, F->dDepth, n * 4, hipMemcpyDeviceToHost, R.stream));
+		HIP_CHECK(hipMemcpyAsync(F->pub.stencil, F->dStencil, n, hipMemcpyDeviceToHost, R.stream));
+	}
 	HIP_CHECK(hipStreamSynchronize(R.stream));
 }
 
@@ -725,6 +748,9 @@ SRPFramebuffer* srpNewFramebuffer(size_t w, size_t h)
 	HIP_CHECK(hipHostMalloc((void**) &F->pub.color, n * 4 + 16, hipHostMallocDefault));
 	HIP_CHECK(hipHostMalloc((void**) &F->pub.depth, n * 4 + 16, hipHostMallocDefault));
 	HIP_CHECK(hipHostMalloc((void**) &F->pub.stencil, n + 16, hipHostMallocDefault));
+	F->hColor = F->pub.color;
+	F->hDepth = F->pub.depth;
+	F->hStencil = F->pub.stencil;
 	HIP_CHECK(hipMalloc((void**) &F->dColor, n * 4 + 16));
 	HIP_CHECK(hipMalloc((void**) &F->dDepth, n * 4 + 16));
 	HIP_CHECK(hipMalloc((void**) &F->dStencil, n + 16));
@@ -784,7 +810,10 @@ void srpFramebufferSetDeferred(const SRPFramebuffer* fb, bool deferred)
 	}
 	FbImpl* F = fbImpl(fb);
 	if (deferred && !F->deferred)
+	{
 		fbUpload(F);
+		HIP_CHECK(hipStreamSynchronize(rt().stream));   /* the host arrays are the caller's again */
+	}
 	if (!deferred && F->deferred)
 		fbDownload(F);
 	F->deferred = deferred;
@@ -1763,7 +1792,10 @@ void drawBuffer(const SRPIndexBuffer* ib, const SRPVertexBuffer* vb, const SRPFr
 	                    (uniformBytes && memcmp(R.sentParams.data() + kTotalsOff, hp + kParamsHead, uniformBytes) != 0);
 	if (resend)
 	{
-		HIP_CHECK(hipMemcpyAsync(R.dParams, &H, paramsBytes, hipMemcpyHostToDevice, R.stream));
+		if (paramsBytes <= UPLOAD_SMALL_BYTES)
+			uploadSmall(R.dParams, &H, paramsBytes, R.stream);
+		else
+			HIP_CHECK(hipMemcpyAsync(R.dParams, &H, paramsBytes, hipMemcpyHostToDevice, R.stream));
 		R.sentParams.assign(hp, hp + kTotalsOff);
 		R.sentParams.insert(R.sentParams.end(), hp + kParamsHead, hp + kParamsHead + uniformBytes);
 	}
