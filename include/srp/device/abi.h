@@ -11,7 +11,7 @@
 #include <stdint.h>
 #include "srp/context.h"
 
-#define SRP_ABI_VERSION 18u
+#define SRP_ABI_VERSION 19u
 #define SRP_MAX_VARYINGS 16
 #define SRP_MAX_WORDS 32          /* fast interpolation path: 4-byte words */
 #define SRP_MAX_VARYING_BYTES 256 /* general path: bytes per fragment */
@@ -184,10 +184,11 @@ typedef struct SrpRasterLaunch
 {
 	const SrpDrawParams* params;
 	const SrpTri* tris;
-	const uint32_t* tileList;   /* pair indices, grouped by tile, in primitive order */
+	const uint32_t* tileList;   /* grouped by tile, in primitive order: a triangle record, whose
+	                               coverage is not known, or 0x80000000 | the index of a pair */
 	const uint32_t* tileStart;  /* first list entry of each tile */
 	const uint32_t* tileEnd;    /* one past its last entry (start == end: empty) */
-	const uint32_t* pairRec;    /* triangle record of a pair | 0x80000000 if pairMask is exact */
+	const uint32_t* pairRec;    /* triangle record of a pair; 0xFFFFFFFF: none, its mask is 0 */
 	const unsigned long long* pairMask;  /* exact coverage of the tile's 8x8 pixels */
 	uint32_t nTiles;
 	uint32_t lateZ;

@@ -567,10 +567,11 @@ __device__ __forceinline__ void rasterTileSimple(const SrpRasterLaunch& L, const
 
 	for (uint32_t i = begin; i < end; i++)
 	{
-		const uint32_t pr = L.pairRec[L.tileList[i]];
+		const uint32_t entry = L.tileList[i];
+		const uint32_t pr = entry >> 31 ? L.pairRec[entry & 0x7FFFFFFFu] : entry;
 		if (pr == 0xFFFFFFFFu)   /* a pair without a record (a batch's capacity exceeded) covers nothing */
 			continue;
-		const SrpTri* T = &L.tris[pr & 0x7FFFFFFFu];
+		const SrpTri* T = &L.tris[pr];
 		if (!(px >= (int) T->x0 && px < (int) T->x1 && py >= (int) T->y0 && py < (int) T->y1))
 			continue;
 		const int ny = py - (int) T->y0, nx = px - (int) T->x0;
@@ -969,12 +970,12 @@ __device__ __forceinline__ void rasterTileBatched(const SrpRasterLaunch& L, cons
 		const bool fresh = mine >= filled && mine < avail;
 		if (fresh)
 		{
-			const uint32_t pi = L.tileList[i + mine];
-			const uint32_t pr = L.pairRec[pi];
-			sknown = (pr >> 31) != 0;
+			const uint32_t entry = L.tileList[i + mine], pi = entry & 0x7FFFFFFFu;
+			sknown = (entry >> 31) != 0;
+			const uint32_t pr = sknown ? L.pairRec[pi] : pi;
 			smask = sknown ? L.pairMask[pi] : 0ull;
 			if (pr != 0xFFFFFFFFu)   /* a pair without a record (capacity exceeded) covers nothing */
-				recIdx[lane] = pr & 0x7FFFFFFFu;
+				recIdx[lane] = pr;
 		}
 		__syncthreads();
 		/* Triangles without an exact mask: pixel-parallel coverage, 8

@@ -547,9 +547,12 @@ __device__ __forceinline__ void fanTriangle(const AsmArgs& A, const AsmDraw& W, 
 				if (o < A.itemCap)
 				{
 					A.pairKeys[o] = key;
-					A.pairVals[o] = o;
-					A.pairRec[o] = fits ? (r | (known ? 0x80000000u : 0u)) : 0xFFFFFFFFu;
-					A.pairMask[o] = fits ? m : 0ull;
+					A.pairVals[o] = fits && !known ? r : (o | 0x80000000u);
+					if (known || !fits)
+					{
+						A.pairRec[o] = fits ? r : 0xFFFFFFFFu;
+						A.pairMask[o] = fits ? m : 0ull;
+					}
 				}
 				o++;
 			});
@@ -730,8 +733,8 @@ __device__ __forceinline__ void fillRows(const AsmArgs& A, const AsmDraw& W, uin
 				if (o < A.itemCap)
 				{
 					A.pairKeys[o] = W.tileBase + ty * P->tilesX + tx0 + gl;
-					A.pairVals[o] = o;
-					A.pairRec[o] = fits ? (recBase | 0x80000000u) : 0xFFFFFFFFu;
+					A.pairVals[o] = o | 0x80000000u;
+					A.pairRec[o] = fits ? recBase : 0xFFFFFFFFu;
 					A.pairMask[o] = fits ? m : 0ull;
 				}
 			}
@@ -1089,8 +1092,8 @@ __device__ __forceinline__ void clipFillFans(const AsmArgs& A, const AsmDraw& W,
 			{
 				const uint32_t q = (uint32_t) at;
 				A.pairKeys[q] = key;
-				A.pairVals[q] = q;
-				A.pairRec[q] = oFits ? (oRec | 0x80000000u) : 0xFFFFFFFFu;
+				A.pairVals[q] = q | 0x80000000u;
+				A.pairRec[q] = oFits ? oRec : 0xFFFFFFFFu;
 				A.pairMask[q] = oFits ? m : 0ull;
 			}
 			if (at + weight > A.itemCap)
@@ -1578,8 +1581,8 @@ __global__ __launch_bounds__(128) void k_assemble_points(AsmArgs A)
  * span at a time.  Lane r finds the tiles of tile row r (64 rows a round),
  * then the lanes take the listed tiles in order, each finding its row by
  * bisection over the rows' running counts, so that consecutive items are
- * written together.  (Pairs without masks: pairMask is only read for a pair
- * marked exact, or one without a record, whose mask is zero.) */
+ * written together.  (Pairs without masks: a record's list entry is the
+ * record itself.) */
 __global__ __launch_bounds__(256) void k_expand_spans(const SrpSpan* spans, const SrpTri* tris, const uint32_t* count,
                                                       uint32_t cap, uint32_t* pairKeys, uint32_t* pairVals,
                                                       uint32_t* pairRec, unsigned long long* pairMask, uint32_t itemCap)
@@ -1604,7 +1607,7 @@ __global__ __launch_bounds__(256) void k_expand_spans(const SrpSpan* spans, cons
 				if (o >= itemCap)
 					break;
 				pairKeys[o] = sp.tileBase;
-				pairVals[o] = o;
+				pairVals[o] = o | 0x80000000u;
 				pairRec[o] = 0xFFFFFFFFu;
 				pairMask[o] = 0ull;
 			}
@@ -1643,8 +1646,7 @@ __global__ __launch_bounds__(256) void k_expand_spans(const SrpSpan* spans, cons
 				if (k < total && o < itemCap)
 				{
 					pairKeys[o] = key;
-					pairVals[o] = o;
-					pairRec[o] = sp.rec;
+					pairVals[o] = sp.rec;
 				}
 			}
 			item += total;

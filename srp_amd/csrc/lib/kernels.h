@@ -71,9 +71,10 @@ struct AsmArgs
 	SrpLine* lines;
 	SrpPoint* points;
 	uint32_t* pairKeys;       /* tile of each (tile, triangle) pair */
-	uint32_t* pairVals;       /* pair index (sorted along with the keys) */
-	uint32_t* pairRec;        /* triangle record | 0x80000000 when the mask is exact */
-	unsigned long long* pairMask; /* coverage of the tile's 64 pixels */
+	uint32_t* pairVals;       /* list entry, sorted along with the keys: a pair without a mask is its
+	                             triangle record; with one, the pair's index | 0x80000000 */
+	uint32_t* pairRec;        /* pairs with masks: triangle record, or 0xFFFFFFFF (none: mask 0) */
+	unsigned long long* pairMask; /* and the exact coverage of the tile's 64 pixels */
 	SrpFrag* frags;
 	uint32_t* fragKeys;
 	uint8_t* genVaryings;
@@ -173,12 +174,12 @@ void tileBounds(const uint32_t* keys, size_t n, uint32_t* start, uint32_t* end, 
                 const uint32_t* nDev = nullptr);
 
 /* Stable sort of the first min(cap, *nDev) items by tile (bits <= 16 bits of
- * the keys, which fit them) in one launch: order[i] is the index of the item
+ * the keys, which fit them) in one launch: sorted[i] is the value of the item
  * at place i; start and end of each tile that received one are set.  cap <=
- * TS_MAX_ITEMS. */
+ * TS_MAX_ITEMS; sorted is not vals. */
 constexpr uint32_t TS_MAX_ITEMS = 16384;
-void tileSort(const uint32_t* keys, size_t cap, int bits, uint32_t* order, uint32_t* start, uint32_t* end, hipStream_t s,
-              const uint32_t* nDev);
+void tileSort(const uint32_t* keys, const uint32_t* vals, size_t cap, int bits, uint32_t* sorted, uint32_t* start,
+              uint32_t* end, hipStream_t s, const uint32_t* nDev);
 
 struct SortScratch
 {
@@ -192,9 +193,11 @@ struct SortScratch
 /* Stable LSD radix sort of (keys, vals) on the low `bits` bits of the keys.
  * The sorted arrays are returned through *outKeys / *outVals (either the
  * inputs or the scratch buffers).  With nDev, n is a capacity and the count
- * is min(n, *nDev), read on the device (no host synchronisation). */
+ * is min(n, *nDev), read on the device (no host synchronisation).  With
+ * index, the values are the items' indices: vals need not hold them. */
 void radixSort(uint32_t* keys, uint32_t* vals, size_t n, int bits, SortScratch& scratch,
-               uint32_t** outKeys, uint32_t** outVals, hipStream_t s, const uint32_t* nDev = nullptr);
+               uint32_t** outKeys, uint32_t** outVals, hipStream_t s, const uint32_t* nDev = nullptr,
+               bool index = false);
 void radixSortReserve(SortScratch& scratch, size_t n);
 
 /* 16 words of a draw's counter block copied to host-mapped memory

@@ -1150,14 +1150,15 @@ void srp_lib_tile_sort(const uint32_t* keys, size_t cap, size_t count, uint32_t 
 		return;
 	Runtime& R = rt();
 	uint32_t* d = nullptr;
-	const size_t words = 2 * cap + 2 * (size_t) nTiles + 1;
+	const size_t words = 3 * cap + 2 * (size_t) nTiles + 1;
 	HIP_CHECK(hipMalloc((void**) &d, words * sizeof(uint32_t) + 16));
-	uint32_t *dk = d, *dOrd = d + cap, *dRange = d + 2 * cap, *dn = dRange + 2 * (size_t) nTiles;
+	uint32_t *dk = d, *dv = d + cap, *dOrd = d + 2 * cap, *dRange = d + 3 * cap, *dn = dRange + 2 * (size_t) nTiles;
 	const uint32_t count32 = (uint32_t) count;
 	HIP_CHECK(hipMemcpyAsync(dk, keys, cap * sizeof(uint32_t), hipMemcpyHostToDevice, R.stream));
 	HIP_CHECK(hipMemcpyAsync(dn, &count32, sizeof(uint32_t), hipMemcpyHostToDevice, R.stream));
 	fillU32(dRange, 0u, 2 * (size_t) nTiles, R.stream);
-	tileSort(dk, cap, bits, dOrd, dRange, dRange + nTiles, R.stream, dn);
+	iota(dv, cap, R.stream);
+	tileSort(dk, dv, cap, bits, dOrd, dRange, dRange + nTiles, R.stream, dn);
 	HIP_CHECK(hipMemcpyAsync(order, dOrd, count * sizeof(uint32_t), hipMemcpyDeviceToHost, R.stream));
 	HIP_CHECK(hipMemcpyAsync(start, dRange, nTiles * sizeof(uint32_t), hipMemcpyDeviceToHost, R.stream));
 	HIP_CHECK(hipMemcpyAsync(end, dRange + nTiles, nTiles * sizeof(uint32_t), hipMemcpyDeviceToHost, R.stream));
@@ -1378,7 +1379,9 @@ void enqueueEmit(Runtime& R, const FitCaps& want, bool speculative)
 		A.fragKeys = (uint32_t*) take(R.fragKeys, want.items, 4, 16, caps.items);
 		caps.spans = 0;
 	}
-	uint32_t* order = (D.backend != 0) ? (uint32_t*) take(R.order, want.items, 4, 16, caps.items) : nullptr;
+	const int tileBits = bitsFor(D.nTiles);
+	const bool oneSort = D.backend == 0 && want.items <= TS_MAX_ITEMS && tileBits <= 16;
+	uint32_t* order = (D.backend != 0 || oneSort) ? (uint32_t*) take(R.order, want.items, 4, 16, caps.items) : nullptr;
 	/* the sort, tile ranges, span and fragment kernels size their grids by these */
 	caps.items = std::min(caps.items, want.items);
 	caps.spans = std::min(caps.spans, want.spans);
@@ -1415,10 +1418,9 @@ void enqueueEmit(Runtime& R, const FitCaps& want, bool speculative)
 	{
 		/* spans: the grid strides over the device-side count */
 		launchExpandSpans(A, (uint32_t) std::min<unsigned long long>((caps.spans + 3) / 4, 2048ull), R.stream);
-		uint32_t *keys, *vals = A.pairVals;
-		const int tileBits = bitsFor(D.nTiles);
-		if (caps.items <= TS_MAX_ITEMS && tileBits <= 16)
-			tileSort(A.pairKeys, caps.items, tileBits, vals, tileStart, tileEnd, R.stream, items);
+		uint32_t *keys, *vals = order;
+		if (oneSort)
+			tileSort(A.pairKeys, A.pairVals, caps.items, tileBits, vals, tileStart, tileEnd, R.stream, items);
 		else
 		{
 			radixSort(A.pairKeys, A.pairVals, caps.items, tileBits, R.sort, &keys, &vals, R.stream, items);
@@ -1453,9 +1455,8 @@ void enqueueEmit(Runtime& R, const FitCaps& want, bool speculative)
 	}
 	else
 	{
-		iota(order, caps.items, R.stream);
 		uint32_t *keys, *vals;
-		radixSort(A.fragKeys, order, caps.items, D.fragBits, R.sort, &keys, &vals, R.stream, items);
+		radixSort(A.fragKeys, order, caps.items, D.fragBits, R.sort, &keys, &vals, R.stream, items, true);
 		SrpFragLaunch fl;
 		memset(&fl, 0, sizeof(fl));
 		fl.params = R.dParams;

@@ -16,7 +16,7 @@
 namespace srp {
 namespace lib {
 
-/* Record indices carry a flag in bit 31 of the tile pairs' record word;
+/* A tile list's entry is a record index, or a pair index with bit 31 set;
  * list indices and tile ranges are 32-bit.  2^31 - 1 items of 28 bytes
  * (pair key, value, record, mask, sort copies) is already ~60 GB. */
 constexpr uint64_t kMaxDrawRecords = 0x7FFFFFFFull;

@@ -3,6 +3,8 @@
  * lists), fills. */
 #include "kernels.h"
 
+#include <algorithm>
+
 namespace srp {
 namespace lib {
 
@@ -291,20 +293,52 @@ void scanExclusiveMulti(uint32_t* base, size_t stride, int nArrays, size_t n, ui
 }
 
 /* Tile ranges of a list sorted by tile: [start, end) per tile; tiles that
- * received nothing keep start == end == 0 (set by the caller's fill). */
-__global__ void k_tile_bounds(const uint32_t* keys, size_t n, const uint32_t* nDev, uint32_t* start, uint32_t* end)
+ * received nothing keep start == end == 0 (set by the caller's fill).  A
+ * thread takes EACH items: four from one load where the list is long (92 M
+ * items: 188 us with one each, 96 with four), one where it is short and the
+ * threads few (350 k items: 2.6 and 3.7 us). */
+constexpr size_t TB_LONG_FROM = (size_t) 4 << 20;
+
+template <int EACH>
+__global__ __launch_bounds__(256) void k_tile_bounds(const uint32_t* keys, size_t n, const uint32_t* nDev,
+                                                     uint32_t* start, uint32_t* end)
 {
 	if (nDev && *nDev < n) n = *nDev;
-	const size_t i = (size_t) blockIdx.x * blockDim.x + threadIdx.x;
+	const size_t i = ((size_t) blockIdx.x * 256u + threadIdx.x) * EACH;
 	if (i >= n) return;
-	const uint32_t k = keys[i];
-	if (i == 0 || keys[i - 1] != k) start[k] = (uint32_t) i;
-	if (i + 1 == n || keys[i + 1] != k) end[k] = (uint32_t) (i + 1);
+	uint32_t k[EACH + 2];   /* items i - 1 .. i + EACH */
+	k[0] = i ? keys[i - 1] : 0u;
+	if (EACH == 4 && i + EACH <= n)
+	{
+		const uint4 v = *reinterpret_cast<const uint4*>(keys + i);
+		k[1] = v.x;
+		k[EACH > 1 ? 2 : 1] = v.y;
+		k[EACH > 1 ? 3 : 1] = v.z;
+		k[EACH > 1 ? 4 : 1] = v.w;
+	}
+	else
+	{
+#pragma unroll
+		for (int q = 0; q < EACH; q++)
+			k[1 + q] = i + (size_t) q < n ? keys[i + (size_t) q] : 0u;
+	}
+	k[EACH + 1] = i + EACH < n ? keys[i + EACH] : 0u;
+#pragma unroll
+	for (int q = 0; q < EACH; q++)
+		if (i + (size_t) q < n)
+		{
+			const size_t at = i + (size_t) q;
+			if (at == 0 || k[q] != k[q + 1]) start[k[q + 1]] = (uint32_t) at;
+			if (at + 1 == n || k[q + 2] != k[q + 1]) end[k[q + 1]] = (uint32_t) (at + 1);
+		}
 }
 
 void tileBounds(const uint32_t* keys, size_t n, uint32_t* start, uint32_t* end, hipStream_t s, const uint32_t* nDev)
 {
-	if (n) hipLaunchKernelGGL(k_tile_bounds, dim3((uint32_t) ((n + 255) / 256)), dim3(256), 0, s, keys, n, nDev, start, end);
+	if (n > TB_LONG_FROM)
+		hipLaunchKernelGGL(k_tile_bounds<4>, dim3((uint32_t) ((n + 1023) / 1024)), dim3(256), 0, s, keys, n, nDev, start, end);
+	else if (n)
+		hipLaunchKernelGGL(k_tile_bounds<1>, dim3((uint32_t) ((n + 255) / 256)), dim3(256), 0, s, keys, n, nDev, start, end);
 }
 
 /* ------------------------------------------------------------ radix sort */
@@ -313,17 +347,22 @@ constexpr int RS_THREADS = 256;
 constexpr int RS_SLICES = 2;     /* slices of RS_THREADS items ranked per round */
 constexpr int RS_CHUNK = 1024;   /* items per block: more blocks than CUs for the 1080p mesh's ~350 k pairs
                                    (measured: 4096 0.234 ms/frame, 2048 0.223, 1024 0.219) */
-/* Items per block of a sort of more than RS_LONG_FROM items: each block
- * then writes longer runs per digit (RS_LONG_CHUNK / 256 keys on average,
- * whole cache lines rather than pieces of them), the digit counts to scan
- * shrink by the same factor, and there are still thousands of blocks. */
+/* A sort of more than RS_LONG_FROM items takes whole rounds of
+ * RS_LONG_ROUND items a block (k_radix_scatter_long), some RS_LONG_BLOCKS
+ * blocks of at most RS_LONG_CHUNK: enough to fill the chip several times
+ * over, and few enough digit counts to scan. */
+constexpr int RS_LONG_ROUND = 4096;
 constexpr int RS_LONG_CHUNK = 32768;
-constexpr size_t RS_LONG_FROM = (size_t) 4 << 20;
+constexpr int RS_LONG_BLOCKS = 2048;
+constexpr size_t RS_LONG_FROM = (size_t) 1 << 20;
 
 /* The block size a sort of n items uses (identical for its reservation). */
 inline uint32_t rsChunk(size_t n)
 {
-	return n > RS_LONG_FROM ? (uint32_t) RS_LONG_CHUNK : (uint32_t) RS_CHUNK;
+	if (n <= RS_LONG_FROM)
+		return (uint32_t) RS_CHUNK;
+	const size_t rounds = (n / RS_LONG_BLOCKS + RS_LONG_ROUND - 1) / RS_LONG_ROUND;
+	return (uint32_t) std::min<size_t>(rounds * RS_LONG_ROUND, RS_LONG_CHUNK);
 }
 
 /* Up to this many blocks, each scatter block sums the per-block digit counts
@@ -342,7 +381,8 @@ constexpr uint32_t RS_GROUP_WORDS = RS_FUSED_MAX_BLOCKS / RS_GROUP * 256u;
 
 /* Digit counts of one block of `chunk` keys, written at
  * hist[digit * digitStride + block * blockStride]; with grp, also added to
- * the block's group row. */
+ * the block's group row.  A thread has RS_HIST_AHEAD keys in flight. */
+constexpr int RS_HIST_AHEAD = 4;
 __global__ __launch_bounds__(RS_THREADS) void k_radix_hist(const uint32_t* keys, size_t n, const uint32_t* nDev,
                                                            uint32_t shift, uint32_t* hist, uint32_t digitStride,
                                                            uint32_t blockStride, uint32_t chunk, uint32_t* grp)
@@ -354,8 +394,17 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_hist(const uint32_t* keys,
 	__syncthreads();
 	const size_t begin = (size_t) blockIdx.x * chunk;
 	const size_t end = (begin + chunk < n) ? begin + chunk : n;
-	for (size_t i = begin + t; i < end; i += RS_THREADS)
-		atomicAdd(&h[(keys[i] >> shift) & 255u], 1u);
+	for (size_t i = begin + t; i < end; i += RS_THREADS * RS_HIST_AHEAD)
+	{
+		uint32_t k[RS_HIST_AHEAD];
+#pragma unroll
+		for (int q = 0; q < RS_HIST_AHEAD; q++)
+			k[q] = i + (size_t) q * RS_THREADS < end ? keys[i + (size_t) q * RS_THREADS] : 0u;
+#pragma unroll
+		for (int q = 0; q < RS_HIST_AHEAD; q++)
+			if (i + (size_t) q * RS_THREADS < end)
+				atomicAdd(&h[(k[q] >> shift) & 255u], 1u);
+	}
 	__syncthreads();
 	hist[(size_t) t * digitStride + (size_t) blockIdx.x * blockStride] = h[t];
 	if (grp && h[t])
@@ -472,7 +521,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter(const uint32_t* ke
 			if (valid[sl])
 			{
 				key[sl] = keysIn[i];
-				val[sl] = valsIn[i];
+				val[sl] = valsIn ? valsIn[i] : (uint32_t) i;
 				d[sl] = (key[sl] >> shift) & 255u;
 			}
 		}
@@ -521,6 +570,126 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter(const uint32_t* ke
 			grp[i] = 0u;
 		if (t == 0)
 			grp[RS_GROUP_WORDS] = 0u;
+	}
+}
+
+/* The scatter of a long sort (hist: the exclusive scan of the digit-major
+ * counts).  A round's 4,096 items are put in digit order in LDS first, so
+ * that they leave in runs of sixteen a digit on average, whole lines where
+ * one item at a time would write each line in pieces, from several rounds,
+ * with more lines open than the L2s hold.  A wave ranks 1,024 consecutive
+ * items, 64 at a time, as k_tile_sort does.
+ * The binning of a 1920x1080 mix, 73 M pairs a pass: 1,200 us with the short
+ * rounds' scatter, 440 so (550 where the digits are the tiles' low bits). */
+constexpr int RS_LONG_EACH = RS_LONG_ROUND / RS_THREADS;
+
+__global__ __launch_bounds__(RS_THREADS) void k_radix_scatter_long(const uint32_t* __restrict__ keysIn,
+                                                                   const uint32_t* __restrict__ valsIn,
+                                                                   uint32_t* __restrict__ keysOut,
+                                                                   uint32_t* __restrict__ valsOut, size_t n,
+                                                                   const uint32_t* nDev, uint32_t shift,
+                                                                   const uint32_t* __restrict__ hist, uint32_t nBlocks,
+                                                                   uint32_t chunk)
+{
+	if (nDev && *nDev < n) n = *nDev;
+	const size_t begin = (size_t) blockIdx.x * chunk;
+	if (begin >= n)
+		return;
+	__shared__ uint32_t sortedKey[RS_LONG_ROUND], sortedVal[RS_LONG_ROUND];
+	__shared__ uint32_t cnt[4][256];
+	__shared__ uint32_t placeOf[256];   /* digit: its first output place less its first place in the round */
+	__shared__ uint32_t waveSum[4];
+	const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+	const uint64_t below = (1ull << lane) - 1ull;
+	const size_t end = (begin + chunk < n) ? begin + chunk : n;
+	uint32_t running = hist[(size_t) t * nBlocks + blockIdx.x];   /* digit t's next output place */
+	for (size_t base = begin; base < end; base += RS_LONG_ROUND)
+	{
+		const uint32_t have = (uint32_t) (end - base < (size_t) RS_LONG_ROUND ? end - base : (size_t) RS_LONG_ROUND);
+		const uint32_t first = wave * (RS_LONG_ROUND / 4) + lane;
+		uint32_t key[RS_LONG_EACH], val[RS_LONG_EACH], place[RS_LONG_EACH];
+#pragma unroll
+		for (int k = 0; k < RS_LONG_EACH; k++)
+		{
+			const uint32_t i = first + 64u * (uint32_t) k;
+			key[k] = i < have ? keysIn[base + i] : 0u;
+			val[k] = valsIn ? (i < have ? valsIn[base + i] : 0u) : (uint32_t) (base + i);
+		}
+#pragma unroll
+		for (int d = 0; d < 4; d++)
+			cnt[wave][lane + 64u * (uint32_t) d] = 0u;
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+		for (int k = 0; k < RS_LONG_EACH; k++)
+		{
+			const bool valid = first + 64u * (uint32_t) k < have;
+			const uint32_t d = (key[k] >> shift) & 255u;
+			uint64_t peers = __ballot(valid);
+#pragma unroll
+			for (int b = 0; b < 8; b++)
+			{
+				const bool bit = (d >> b) & 1u;
+				const uint64_t m = __ballot(bit);
+				peers &= bit ? m : ~m;
+			}
+			const uint32_t rank = (uint32_t) __popcll(peers & below);
+			const uint32_t before = cnt[wave][d];
+			place[k] = before + rank;
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			if (valid && rank == 0)
+				cnt[wave][d] = before + (uint32_t) __popcll(peers);
+			__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		}
+		__syncthreads();
+		uint32_t sum = 0, c[4];
+#pragma unroll
+		for (int w = 0; w < 4; w++)
+		{
+			c[w] = sum;
+			sum += cnt[w][t];
+		}
+		uint32_t incl = sum;
+#pragma unroll
+		for (uint32_t off = 1; off < 64; off <<= 1)
+		{
+			const uint32_t v = __shfl_up(incl, off);
+			if (lane >= off) incl += v;
+		}
+		if (lane == 63u)
+			waveSum[wave] = incl;
+		__syncthreads();
+		uint32_t at = incl - sum;   /* digit t's first place in the round */
+		for (uint32_t w = 0; w < wave; w++)
+			at += waveSum[w];
+#pragma unroll
+		for (int w = 0; w < 4; w++)
+			cnt[w][t] = at + c[w];
+		placeOf[t] = running - at;
+		running += sum;
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < RS_LONG_EACH; k++)
+			if (first + 64u * (uint32_t) k < have)
+			{
+				const uint32_t p = cnt[wave][(key[k] >> shift) & 255u] + place[k];
+				sortedKey[p] = key[k];
+				sortedVal[p] = val[k];
+			}
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < RS_LONG_EACH; k++)
+		{
+			const uint32_t p = t + RS_THREADS * (uint32_t) k;
+			if (p < have)
+			{
+				const uint32_t key1 = sortedKey[p];
+				const uint32_t dst = placeOf[(key1 >> shift) & 255u] + p;
+				keysOut[dst] = key1;
+				valsOut[dst] = sortedVal[p];
+			}
+		}
+		/* the next round's writes of cnt follow this round's reads of it by
+		 * two barriers, those of the sorted items by three */
 	}
 }
 
@@ -574,7 +743,7 @@ void radixSortReserve(SortScratch& sc, size_t n)
 		sc.histCap = (histN + 1) * 2;
 		hipMalloc(&sc.hist, sc.histCap * sizeof(uint32_t));
 	}
-	if (nBlocks > RS_FUSED_MAX_BLOCKS)
+	if (nBlocks > RS_FUSED_MAX_BLOCKS || chunk != (uint32_t) RS_CHUNK)
 		scanReserve(sc.scan, histN, 1);
 	else if (!sc.grp)
 	{
@@ -587,12 +756,16 @@ void radixSortReserve(SortScratch& sc, size_t n)
 }
 
 void radixSort(uint32_t* keys, uint32_t* vals, size_t n, int bits, SortScratch& sc,
-               uint32_t** outKeys, uint32_t** outVals, hipStream_t s, const uint32_t* nDev)
+               uint32_t** outKeys, uint32_t** outVals, hipStream_t s, const uint32_t* nDev, bool index)
 {
 	*outKeys = keys;
 	*outVals = vals;
 	if (n <= 1 || bits <= 0)
+	{
+		if (index)
+			iota(vals, n, s);
 		return;
+	}
 	const uint32_t chunk = rsChunk(n);
 	const uint32_t nBlocks = (uint32_t) ((n + chunk - 1) / chunk);
 	radixSortReserve(sc, n);
@@ -601,14 +774,15 @@ void radixSort(uint32_t* keys, uint32_t* vals, size_t n, int bits, SortScratch& 
 	uint32_t* vIn = vals;
 	uint32_t* kOut = sc.keys;
 	uint32_t* vOut = sc.vals;
-	const bool fused = nBlocks <= RS_FUSED_MAX_BLOCKS;
+	const bool fused = nBlocks <= RS_FUSED_MAX_BLOCKS && chunk == (uint32_t) RS_CHUNK;
 	for (int shift = 0; shift < bits; shift += 8)
 	{
+		const uint32_t* from = index && shift == 0 ? nullptr : vIn;
 		if (fused)
 		{
 			hipLaunchKernelGGL(k_radix_hist, dim3(nBlocks), dim3(RS_THREADS), 0, s, kIn, n, nDev, (uint32_t) shift,
 			                   sc.hist, 1u, 256u, chunk, sc.grp);
-			hipLaunchKernelGGL(k_radix_scatter<true>, dim3(nBlocks), dim3(RS_THREADS), 0, s, kIn, vIn, kOut, vOut, n,
+			hipLaunchKernelGGL(k_radix_scatter<true>, dim3(nBlocks), dim3(RS_THREADS), 0, s, kIn, from, kOut, vOut, n,
 			                   nDev, (uint32_t) shift, sc.hist, nBlocks, chunk, sc.grp);
 		}
 		else
@@ -616,8 +790,12 @@ void radixSort(uint32_t* keys, uint32_t* vals, size_t n, int bits, SortScratch& 
 			hipLaunchKernelGGL(k_radix_hist, dim3(nBlocks), dim3(RS_THREADS), 0, s, kIn, n, nDev, (uint32_t) shift,
 			                   sc.hist, nBlocks, 1u, chunk, (uint32_t*) nullptr);
 			scanExclusiveMulti(sc.hist, histN, 1, histN, sc.hist + histN, sc.scan, s);
-			hipLaunchKernelGGL(k_radix_scatter<false>, dim3(nBlocks), dim3(RS_THREADS), 0, s, kIn, vIn, kOut, vOut, n,
-			                   nDev, (uint32_t) shift, sc.hist, nBlocks, chunk, (uint32_t*) nullptr);
+			if (chunk == (uint32_t) RS_CHUNK)
+				hipLaunchKernelGGL(k_radix_scatter<false>, dim3(nBlocks), dim3(RS_THREADS), 0, s, kIn, from, kOut, vOut,
+				                   n, nDev, (uint32_t) shift, sc.hist, nBlocks, chunk, (uint32_t*) nullptr);
+			else
+				hipLaunchKernelGGL(k_radix_scatter_long, dim3(nBlocks), dim3(RS_THREADS), 0, s, kIn, from, kOut, vOut, n,
+				                   nDev, (uint32_t) shift, sc.hist, nBlocks, chunk);
 		}
 		uint32_t* tk = kIn; kIn = kOut; kOut = tk;
 		uint32_t* tv = vIn; vIn = vOut; vOut = tv;
@@ -627,8 +805,8 @@ void radixSort(uint32_t* keys, uint32_t* vals, size_t n, int bits, SortScratch& 
 }
 
 /* Stable sort by tile of up to TS_MAX_ITEMS items by one block, and the
- * tiles' ranges: order[i] = the item (its index) at place i, start/end of
- * every tile that received one.  An item is one word, tile << 16 | index, so
+ * tiles' ranges: sorted[i] = the value of the item at place i, start/end of
+ * every tile that received one.  Inside, an item is one word, tile << 16 | index, so
  * its radix passes (8 bits each) stay in LDS.  A wave ranks consecutive
  * items, 64 at a time, in order; a digit's places are ordered by wave, then
  * within the wave.
@@ -642,9 +820,10 @@ constexpr int TS_THREADS = 1024;
 constexpr int TS_WAVES = TS_THREADS / 64;
 constexpr int TS_ROUNDS = (int) (TS_MAX_ITEMS / TS_THREADS);
 
-__global__ __launch_bounds__(TS_THREADS) void k_tile_sort(const uint32_t* __restrict__ keys, uint32_t cap,
+__global__ __launch_bounds__(TS_THREADS) void k_tile_sort(const uint32_t* __restrict__ keys,
+                                                          const uint32_t* __restrict__ vals, uint32_t cap,
                                                           const uint32_t* __restrict__ nDev, int bits,
-                                                          uint32_t* __restrict__ order, uint32_t* __restrict__ start,
+                                                          uint32_t* __restrict__ sorted, uint32_t* __restrict__ start,
                                                           uint32_t* __restrict__ end)
 {
 	__shared__ uint32_t item[TS_MAX_ITEMS];
@@ -754,18 +933,19 @@ __global__ __launch_bounds__(TS_THREADS) void k_tile_sort(const uint32_t* __rest
 		if ((uint32_t) k < rounds && i < n)
 		{
 			const uint32_t tile = it[k] >> 16;
-			order[i] = it[k] & 0xFFFFu;
+			sorted[i] = vals[it[k] & 0xFFFFu];
 			if (i == 0 || item[i - 1] >> 16 != tile) start[tile] = i;
 			if (i + 1 == n || item[i + 1] >> 16 != tile) end[tile] = i + 1;
 		}
 	}
 }
 
-void tileSort(const uint32_t* keys, size_t cap, int bits, uint32_t* order, uint32_t* start, uint32_t* end, hipStream_t s,
-              const uint32_t* nDev)
+void tileSort(const uint32_t* keys, const uint32_t* vals, size_t cap, int bits, uint32_t* sorted, uint32_t* start,
+              uint32_t* end, hipStream_t s, const uint32_t* nDev)
 {
 	if (cap)
-		hipLaunchKernelGGL(k_tile_sort, dim3(1), dim3(TS_THREADS), 0, s, keys, (uint32_t) cap, nDev, bits, order, start, end);
+		hipLaunchKernelGGL(k_tile_sort, dim3(1), dim3(TS_THREADS), 0, s, keys, vals, (uint32_t) cap, nDev, bits, sorted,
+		                   start, end);
 }
 
 /* ------------------------------------------------------------------ fills */

@@ -95,3 +95,24 @@ def test_one_launch_tile_sort(cap, count, tiles, kind):
     last = np.searchsorted(keys[:count][want], np.arange(tiles), "right")
     some = last > first
     assert np.array_equal(start, np.where(some, first, 0)) and np.array_equal(end, np.where(some, last, 0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cap,count,bits,kind", [
+    (1 << 20, 1 << 20, 15, "tiles"),                 # the last size of the short rounds
+    ((1 << 20) + 1, (1 << 20) + 1, 15, "tiles"),     # long rounds, the last one of a single item
+    (1_200_000, 4_097, 9, "few"),                    # most blocks past the device count
+    (9_000_000, 8_388_608, 16, "few"),               # blocks of two rounds, very uneven digits
+    (9_000_000, 8_388_607, 21, "uniform"),
+])
+def test_long_sort_matches_stable_argsort(cap, count, bits, kind):
+    lib = ctypes.CDLL(LIB, mode=ctypes.RTLD_LOCAL)
+    lib.srp_lib_radix_sort.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_size_t,
+                                       ctypes.c_int]
+    keys = _keys(np.random.default_rng(22), cap, bits, kind)
+    vals = np.arange(cap, dtype=np.uint32)[::-1].copy()
+    k, v = keys.copy(), vals.copy()
+    lib.srp_lib_radix_sort(k.ctypes.data, v.ctypes.data, cap, count, bits)
+    order = np.argsort(keys[:count] & np.uint32((1 << (8 * ((bits + 7) // 8))) - 1), kind="stable")
+    assert np.array_equal(v[:count], vals[:count][order])
+    assert np.array_equal(k[:count], keys[:count][order])
