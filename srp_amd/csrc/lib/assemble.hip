@@ -935,6 +935,49 @@ __device__ __forceinline__ uint32_t drawOfInput(const AsmDraw* D, uint32_t n, ui
  * the limits below only guard numerically degenerate input. */
 constexpr uint32_t CLIP_GROUP = 16;
 
+/* spanTiles of every fan triangle of a group that is a span, its rows shared
+ * out to the group's lanes: a clipped triangle has few fan triangles, and a
+ * lane each left the others waiting while it went down the view's tile rows
+ * (counting and emitting the clipped of 500,000 triangles over 1920x1080: 777
+ * and 924 us, 707 and 867 so). */
+__device__ __forceinline__ uint32_t groupSpanTiles(const SrpDrawParams* P, const SrpTri& T, bool span, uint32_t gl)
+{
+	const uint32_t sh = P->tileShift;
+	uint32_t todo = (uint32_t) (__ballot(span) >> (__lane_id() & ~(CLIP_GROUP - 1u))) & ((1u << CLIP_GROUP) - 1u);
+	const uint32_t box0 = (uint32_t) T.x0 | ((uint32_t) T.y0 << 16);
+	const uint32_t box1 = (uint32_t) T.x1 | ((uint32_t) T.y1 << 16);
+	uint32_t mine = 0;
+	while (todo)   /* the same for every lane of the group */
+	{
+		const int o = __builtin_ctz(todo);
+		todo &= todo - 1u;
+		float l0[3], dx[3], dy[3];
+#pragma unroll
+		for (int e = 0; e < 3; e++)
+		{
+			l0[e] = __shfl(T.l0[e], o, CLIP_GROUP);
+			dx[e] = __shfl(T.dx[e], o, CLIP_GROUP);
+			dy[e] = __shfl(T.dy[e], o, CLIP_GROUP);
+		}
+		const uint32_t b0 = __shfl(box0, o, CLIP_GROUP), b1 = __shfl(box1, o, CLIP_GROUP);
+		SrpSpanScan S;
+		srpSpanScanInit(&S, l0, dx, dy, (int) (b0 & 0xFFFFu), (int) (b0 >> 16), (int) (b1 & 0xFFFFu), (int) (b1 >> 16));
+		const uint32_t last = ((b1 >> 16) - 1u) >> sh;
+		uint32_t n = 0;
+		for (uint32_t ty = ((b0 >> 16) >> sh) + gl; ty <= last; ty += CLIP_GROUP)
+		{
+			uint32_t x0, x1;
+			if (srpSpanRow(&S, ty, sh, &x0, &x1))
+				n += x1 - x0 + 1u;
+		}
+#pragma unroll
+		for (uint32_t off = 1; off < CLIP_GROUP; off <<= 1)
+			n += __shfl_xor(n, (int) off, CLIP_GROUP);
+		mine = gl == (uint32_t) o ? n : mine;
+	}
+	return mine;
+}
+
 /* The emitting pass of the filled fan triangles of one clipped triangle
  * (polygon mode FILL): set up by their fan lanes, binned by the whole
  * group.  binTriangle scans a box with one lane; here the group's lanes
@@ -957,6 +1000,7 @@ __device__ __forceinline__ void clipFillFans(const AsmArgs& A, const AsmDraw& W,
 	const bool span = ok && isSpan(P, T);
 	const bool boxed = ok && T.x1 > T.x0 && T.y1 > T.y0;
 	const uint32_t sh = P->tileShift;
+	const uint32_t spanPairs = groupSpanTiles(P, T, span, gl);
 	uint32_t nItem = 0;
 	if (span)
 		nItem = 1u;
@@ -1021,6 +1065,7 @@ __device__ __forceinline__ void clipFillFans(const AsmArgs& A, const AsmDraw& W,
 		const uint32_t oflags = __shfl(T.flags, o, CLIP_GROUP);
 		const uint32_t oEx = __shfl(iEx, o, CLIP_GROUP);
 		const bool oSpan = __shfl((int) span, o, CLIP_GROUP) != 0;
+		const uint32_t oPairs = __shfl(spanPairs, o, CLIP_GROUP);
 		const uint32_t oRec = __shfl(r, o, CLIP_GROUP);
 		const bool oFits = __shfl((int) fits, o, CLIP_GROUP) != 0;
 		const int x0 = (int) (ob0 & 0xFFFFu), y0 = (int) (ob0 >> 16);
@@ -1032,11 +1077,7 @@ __device__ __forceinline__ void clipFillFans(const AsmArgs& A, const AsmDraw& W,
 			const uint32_t tx0 = (uint32_t) x0 >> sh, ty0 = (uint32_t) y0 >> sh;
 			const uint32_t ntx = (((uint32_t) x1 - 1u) >> sh) - tx0 + 1u;
 			if (oSpan)
-			{
-				SrpSpanScan S;
-				srpSpanScanInit(&S, l0, dx, dy, x0, y0, x1, y1);
-				weight = srpSpanTiles(&S, sh);
-			}
+				weight = oPairs;
 			else
 			{
 				/* exact masks: tileShift 3 */
@@ -1347,16 +1388,32 @@ __device__ __forceinline__ void clipGroup(const AsmArgs& A, uint32_t g, bool has
 	const bool fan = gl >= 1u && (int) gl + 1 < np;
 	if (EMIT && P->st.polygonMode == SRP_POLYGON_MODE_FILL)
 	{
-		/* (the counting pass keeps one lane per fan triangle: its scan
-		 * stops at a tile's first covered pixel, which for the small
-		 * triangles clipping mostly makes costs less than the group's
-		 * shuffles) */
+		/* (the counting pass keeps one lane per small fan triangle: its
+		 * scan stops at a tile's first covered pixel, which costs less than
+		 * the group's shuffles) */
 		clipFillFans(A, W, gl, a, v, cc, fan, recBase, idBase, itemBase, drop);
 		return;
 	}
 	uint32_t myRec = 0, myItems = 0;
-	if (fan)
-		fanTriangle<false, !EMIT>(A, W, a, v, cc, 0u, 0u, 0u, myRec, myItems, false);
+	if (!EMIT && P->st.polygonMode == SRP_POLYGON_MODE_FILL)
+	{
+		SrpTri T = {};
+		const bool ok = fan && setupTriangle(P, a, v, cc, 0u, T);
+		const bool span = ok && isSpan(P, T);
+		const uint32_t pairs = groupSpanTiles(P, T, span, gl);
+		myRec = ok ? 1u : 0u;
+		if (span)
+		{
+			myItems = pairs;
+			const uint64_t act = __ballot(1);
+			if (__lane_id() == (uint32_t) __builtin_ctzll(act))
+				atomicAdd(A.spanCount, (uint32_t) __popcll(act));
+		}
+		else if (ok)
+			myItems = binTriangle<false>(P, T, 0u, [](uint32_t, uint64_t, bool) {});
+	}
+	else if (fan)
+		fanTriangle<false, false>(A, W, a, v, cc, 0u, 0u, 0u, myRec, myItems, false);
 	/* exclusive scans over the group (items saturate: see fanTriangle) */
 	uint32_t exRec = myRec;
 	unsigned long long exItems = myItems;
@@ -1665,16 +1722,19 @@ void launchClipped(const AsmArgs& A, bool emit, hipStream_t s, uint32_t clipped,
 {
 	const uint32_t blocks = A.nBlocks;
 	if (!blocks) return;
+	/* at most 8,192 blocks: what the chip holds at once (2,048) left it idle
+	 * at the end, some groups having much more to do (the figures above: 707
+	 * and 867 us, 676 and 714 so) */
 	uint32_t clipBlocks;
 	if (clipped != kClipUnknown)
 	{
 		const uint32_t need = (uint32_t) (((uint64_t) clipped + 7u) / 8u);
-		clipBlocks = need < 2048u ? need : 2048u;
+		clipBlocks = need < 8192u ? need : 8192u;
 	}
 	else
 	{
 		const uint64_t want = ((uint64_t) clipHint + clipHint / 4u + 7u) / 8u;
-		clipBlocks = (uint32_t) (want < 256u ? 256u : (want > 2048u ? 2048u : want));
+		clipBlocks = (uint32_t) (want < 256u ? 256u : (want > 8192u ? 8192u : want));
 		/* (a group per triangle of a draw that clips much of its few
 		 * inputs: limited to the main grid, 2,000 triangles of which half
 		 * are clipped took eight rounds, 117 + 144 us; 52 + 36 with a group each) */
