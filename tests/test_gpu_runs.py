@@ -127,3 +127,32 @@ def test_repeated_small_draws_do_not_change_the_frame(cases, n):
             got = [x.copy() for x in s.images]
             for x, y in zip(frames.setdefault(name, got), got):
                 assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
+@pytest.mark.parametrize("w,h", [(16, 8), (40, 128), (24, 136), (64, 1032)])
+def test_clipped_spans_in_one_draw_equal_single_draws(cases, w, h):
+    """Triangles that reach over the view on every side: fans of several
+    spans each, over fewer tile rows than a group has lanes, as many, one
+    more, and many times as many."""
+    a = cases.api()
+    a.NewContext(a.context)
+    a.DepthTest(True)
+    a.DepthCompareOp(cases.CMP_LESS)
+    s = cases.State("test")
+    n = 60
+    rng = np.random.default_rng(h)
+    v = np.concatenate([rng.uniform(-5, 5, (n, 3, 2)), rng.uniform(-1.5, 1.5, (n, 3, 1)), rng.random((n, 3, 3))], -1)
+    v[0, :, :3] = [[-4, -4, 0.9], [4, -4, 0.9], [0, 5, 0.9]]   # covers the view
+    vb = s.vertices(np.ascontiguousarray(v.reshape(-1, 6), np.float32), 24)
+    p = a.program("sc_vsColorPass", [(3, cases.T_FLOAT, cases.PERSPECTIVE)], "sc_fsColor")
+    fb = s.framebuffer(w, h)
+    frames = []
+    for calls in ([(0, 3 * n)], [(3 * k, 3) for k in range(n)]):
+        cases.start_frame(a, fb)
+        for first, count in calls:
+            a.DrawVertexBuffer(vb, fb, C.byref(p), cases.PRIM_TRIANGLES, first, count)
+        a.FramebufferDownload(fb)
+        frames.append([x.copy() for x in s.images])
+    assert np.count_nonzero(frames[0][0]) > w * h // 2
+    for x, y in zip(*frames):
+        assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
