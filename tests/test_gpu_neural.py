@@ -397,3 +397,27 @@ def test_gradients_match_oracle_across_chunk_counts(nn, chunks):
     finally:
         nn.free_net(net)
         nn.free_ds(ds)
+
+
+@pytest.mark.parametrize("n", [393_215, 393_216, 393_217, 1_572_865])
+def test_inference_in_parts_equals_short_calls(nn, n):
+    """Around the size from which an evaluation runs in two parts, and in
+    three, a part's results copied while the next is evaluated: the same values as evaluations of 65,536
+    samples at a time, called twice (the parts' events are used again)."""
+    F, T = synth(n, 50)
+    ds, small = nn.new_ds(n), nn.new_ds(65_536)
+    net = nn.new_net(7)
+    try:
+        nn.ds_write(ds, F, T)
+        want = []
+        for at in range(0, n, 65_536):
+            m = min(65_536, n - at)
+            nn.ds_write(small, F[at:at + m], T[at:at + m])
+            want.append(nn.infer(net, small, m).copy())
+        want = np.concatenate(want)
+        for _ in range(2):
+            assert np.array_equal(nn.infer(net, ds, n), want)
+    finally:
+        nn.free_net(net)
+        nn.free_ds(small)
+        nn.free_ds(ds)
