@@ -254,6 +254,11 @@ void fillFramebuffers(const FillDesc* desc, uint32_t nDesc, uint32_t blocks, hip
  * (pending deferred fills applied first; a synchronous framebuffer's host
  * arrays are uploaded first). */
 hipStream_t libStream();
+/* The library's second stream, for work that a call orders against libStream
+ * by events (libPartEvent, i < kPartEvents) and waits for before it returns. */
+constexpr int kPartEvents = 8;
+hipStream_t libSideStream();
+hipEvent_t libPartEvent(int i);
 /* Report through the user's message callback (printf-style). */
 void libMessage(SRPMessageType type, SRPMessageSeverity sev, const char* fn, const char* fmt, ...);
 void framebufferDevice(const SRPFramebuffer* fb, uint32_t** color, float** depth, uint8_t** stencil);

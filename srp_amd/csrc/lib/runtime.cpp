@@ -212,6 +212,7 @@ struct Runtime
 	 * published (they follow its uploads on the stream); a parameter patch
 	 * after that (a larger clip-vertex buffer) is waited for with this. */
 	hipEvent_t paramsCopied = nullptr;
+	hipEvent_t partDone[kPartEvents] = {};   /* libPartEvent */
 	/* What the device parameter block holds outside its counters (bytes
 	 * [0, kTotalsOff) and the inline uniform from kParamsHead), so that a
 	 * draw with the same parameters need not send them again; size 0: not
@@ -333,12 +334,15 @@ bool fbOwnArrays(const FbImpl* F)
 	return F->pub.color == F->hColor && F->pub.depth == F->hDepth && F->pub.stencil == F->hStencil;
 }
 
-void fbUpload(FbImpl* F)
+/* waited: the call does not return before the stream has read the arrays.
+ * (A kernel reads them when it runs; a caller that goes on at once keeps the
+ * copy calls.) */
+void fbUpload(FbImpl* F, bool waited)
 {
 	Runtime& R = rt();
 	F->pendColor = F->pendDepth = F->pendStencil = false;  /* the host arrays win */
 	const size_t n = F->pub.size;
-	if (fbOwnArrays(F))
+	if (waited && fbOwnArrays(F))
 	{
 		copyArrays({{F->pub.color, F->pub.depth, F->pub.stencil}, {F->dColor, F->dDepth, F->dStencil}, {n * 4, n * 4, n}},
 		           R.stream);
@@ -429,6 +433,19 @@ hipStream_t libStream()
 	return rt().stream;
 }
 
+hipStream_t libSideStream()
+{
+	return rt().side;
+}
+
+hipEvent_t libPartEvent(int i)
+{
+	hipEvent_t& e = rt().partDone[i];
+	if (!e)
+		HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+	return e;
+}
+
 void libMessage(SRPMessageType type, SRPMessageSeverity sev, const char* fn, const char* fmt, ...)
 {
 	char text[1024];
@@ -446,7 +463,7 @@ void framebufferDevice(const SRPFramebuffer* fb, uint32_t** color, float** depth
 	if (F->deferred)
 		fbFlushFills(F);
 	else
-		fbUpload(F);
+		fbUpload(F, false);
 	if (color) *color = F->dColor;
 	if (depth) *depth = F->dDepth;
 	if (stencil) *stencil = F->dStencil;
@@ -810,10 +827,7 @@ void srpFramebufferSetDeferred(const SRPFramebuffer* fb, bool deferred)
 	}
 	FbImpl* F = fbImpl(fb);
 	if (deferred && !F->deferred)
-	{
-		fbUpload(F);
-		HIP_CHECK(hipStreamSynchronize(rt().stream));   /* the host arrays are the caller's again */
-	}
+		fbUpload(F, false);
 	if (!deferred && F->deferred)
 		fbDownload(F);
 	F->deferred = deferred;
@@ -861,7 +875,7 @@ void srpFramebufferUpload(const SRPFramebuffer* fb)
 		message(SRP_MESSAGE_ERROR, SRP_MESSAGE_SEVERITY_HIGH, __func__, "Invalid framebuffer");
 		return;
 	}
-	fbUpload(fbImpl(fb));
+	fbUpload(fbImpl(fb), true);
 	HIP_CHECK(hipStreamSynchronize(rt().stream));
 }
 
@@ -1767,7 +1781,7 @@ void drawBuffer(const SRPIndexBuffer* ib, const SRPVertexBuffer* vb, const SRPFr
 	/* a deferred framebuffer's pending fill rides along with the vertex
 	 * stage below (nothing before the rasteriser touches the framebuffer) */
 	if (!F->deferred)
-		fbUpload(F);
+		fbUpload(F, true);   /* the draw ends in a download */
 	hipEvent_t evDraw = (R.prof(1) || R.prof(3)) ? R.mark() : nullptr;
 	{
 		AsmDraw& AD = *reinterpret_cast<AsmDraw*>((uint8_t*) R.hParams + kAsmDrawOff);

@@ -29,6 +29,9 @@
 
 using namespace srp::nn;
 using srp::lib::libMessage;
+using srp::lib::kPartEvents;
+using srp::lib::libPartEvent;
+using srp::lib::libSideStream;
 using srp::lib::libStream;
 
 #define NN_CHECK(x)                                                                         \
@@ -725,14 +728,14 @@ struct SRPNeuralDataset
 };
 
 /* Evaluations of at least kInferPartsFrom samples run in parts, the results
- * of each copied to the host (on a stream of its own) while the next is
+ * of each copied to the host (on the second stream) while the next is
  * evaluated.  For 1 M samples the copy's 12.6 MB take 227 us on the link and
  * the evaluation 171: 410 us one after the other, 344 in two parts (345 in
  * four, 376 in eight: a part costs some 20 us of launches and events).
  * 262,144 samples take 116 us whole and 113 in two parts, 131,072 69 and 79. */
 constexpr size_t kInferPartsFrom = 393216;
 constexpr size_t kInferPart = 524288;
-constexpr int kInferMaxParts = 8;
+constexpr int kInferMaxParts = kPartEvents;
 
 static int inferParts(size_t count)
 {
@@ -762,9 +765,6 @@ struct SRPNeuralNet
 	float* grad = nullptr;
 	float* rgb = nullptr;
 	size_t rgbCap = 0;
-	/* srpNeuralNetInfer's results on their way to the host, made on first use */
-	hipStream_t copies = nullptr;
-	hipEvent_t partDone[kInferMaxParts] = {};
 };
 
 namespace {
@@ -1035,10 +1035,6 @@ void srpFreeNeuralNet(SRPNeuralNet* N)
 	                N->rgb, N->view};
 	for (void* b : bufs)
 		if (b) NN_CHECK(hipFree(b));
-	if (N->copies)
-		NN_CHECK(hipStreamDestroy(N->copies));
-	for (hipEvent_t e : N->partDone)
-		if (e) NN_CHECK(hipEventDestroy(e));
 	delete N;
 }
 
@@ -1192,11 +1188,7 @@ void srpNeuralNetInfer(const SRPNeuralNet* Nc, const SRPNeuralDataset* D, size_t
 		N->rgbCap = count;
 	}
 	const int parts = inferParts(count);
-	if (parts > 1 && !N->copies)
-		NN_CHECK(hipStreamCreateWithFlags(&N->copies, hipStreamNonBlocking));
-	for (int i = 0; parts > 1 && i < parts; i++)
-		if (!N->partDone[i])
-			NN_CHECK(hipEventCreateWithFlags(&N->partDone[i], hipEventDisableTiming));
+	hipStream_t copies = parts > 1 ? libSideStream() : s;
 	/* whole waves of samples in every part but the last */
 	const size_t per = (count / (size_t) parts + 63) / 64 * 64;
 	for (int i = 0; i < parts; i++)
@@ -1211,18 +1203,18 @@ void srpNeuralNetInfer(const SRPNeuralNet* Nc, const SRPNeuralDataset* D, size_t
 			hipLaunchKernelGGL(k_infer<false>, dim3(blocks), dim3(64), 0, s, (const SrpNnDevice*) N->view, feat,
 			                   (uint64_t) n, N->rgb + at * 3);
 		if (parts > 1)
-			NN_CHECK(hipEventRecord(N->partDone[i], s));
+			NN_CHECK(hipEventRecord(libPartEvent(i), s));
 	}
 	for (int i = 0; i < parts; i++)
 	{
 		const size_t at = (size_t) i * per, n = i + 1 < parts ? per : count - at;
 		if (parts > 1)
-			NN_CHECK(hipStreamWaitEvent(N->copies, N->partDone[i], 0));
+			NN_CHECK(hipStreamWaitEvent(copies, libPartEvent(i), 0));
 		NN_CHECK(hipMemcpyAsync(rgb + at * 3, N->rgb + at * 3, n * 3 * sizeof(float), hipMemcpyDeviceToHost,
-		                        parts > 1 ? N->copies : s));
+		                        copies));
 	}
 	if (parts > 1)
-		NN_CHECK(hipStreamSynchronize(N->copies));
+		NN_CHECK(hipStreamSynchronize(copies));
 	NN_CHECK(hipStreamSynchronize(s));
 }
 

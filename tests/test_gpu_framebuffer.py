@@ -34,9 +34,13 @@ def test_arrays_survive_the_round_trip(w, h, own):
             address[k] = mine[k].ctypes.data
     views = {k: np.frombuffer((C.c_uint8 * (n * C.sizeof(t))).from_address(address[k]), np.uint8) for k, t in kinds}
     want = {}
+    lib = C.CDLL(os.path.join(REPO, "srp_amd", "libsrp_amd.so"))
+    lib.srpFramebufferUpload.argtypes = [C.c_void_p]
+    a.FramebufferSetDeferred(fb, True)
+    a.FramebufferDownload(fb)
     for k, _ in kinds:
         views[k][:] = want[k] = rng.integers(0, 256, views[k].size, dtype=np.uint8)
-    a.FramebufferSetDeferred(fb, True)      # to the device
+    lib.srpFramebufferUpload(fb)
     for k, _ in kinds:
         views[k][:] = 0
     a.FramebufferDownload(fb)
