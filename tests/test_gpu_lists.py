@@ -76,3 +76,45 @@ def test_one_draw_equals_single_draws(cases, op, n, w, h, kind):
     for one, many in zip(frames[:5], frames[5:]):
         for x, y in zip(one, many):
             assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
+
+
+@pytest.mark.parametrize("order", ["sorted", "mixed"])
+def test_line_draws_equal_the_edges_of_flat_triangles(cases, order):
+    """Lines of 0 to 40 samples and of some hundreds and thousands, in every
+    place of a wave, against the same lines walked by one lane each: the
+    three edges of triangles whose last two corners are one point."""
+    a = cases.api()
+    a.NewContext(a.context)
+    a.DepthTest(True)
+    a.DepthCompareOp(cases.CMP_LEQUAL)
+    s = cases.State("test")
+    w, h = 2048, 32
+    rng = np.random.default_rng(5)
+    length = np.concatenate([np.arange(0, 41), [63, 64, 255, 256, 257, 700, 2000, 2047], rng.integers(0, 60, 120)])
+    if order == "mixed":
+        length = rng.permutation(length)
+    n = len(length)
+    v = np.zeros((n, 2, 8), np.float32)
+    start = rng.uniform(0, np.maximum(w - 1 - length, 1))
+    v[:, 0, 0], v[:, 1, 0] = start / w * 2 - 1, (start + length) / w * 2 - 1
+    v[:, :, 1] = rng.uniform(-0.99, 0.99, (n, 2))
+    v[:, :, 2] = rng.uniform(-0.5, 0.5, (n, 2))
+    v[:, :, 3] = 1
+    v[:, :, 4:6] = rng.random((n, 2, 2))
+    v[:, :, 6] = rng.random((n, 1))
+    edges = v[:, [0, 1, 1, 1, 1, 0]].reshape(-1, 8)
+    corners = v[:, [0, 1, 1]].reshape(-1, 8)
+    p = a.program("sc_vsMix", [(2, cases.T_FLOAT, cases.AFFINE), (1, cases.T_FLOAT, cases.FLAT),
+                               (1, cases.T_UINT32, cases.FLAT)], "sc_fsMix")
+    fb = s.framebuffer(w, h)
+    frames = []
+    for data, prim in ((edges, cases.PRIM_LINES), (corners, cases.PRIM_TRIANGLES)):
+        vb = s.vertices(np.ascontiguousarray(data, np.float32), 32)
+        a.RasterPolygonMode(cases.MODES["line"] if prim == cases.PRIM_TRIANGLES else cases.MODES["fill"])
+        cases.start_frame(a, fb)
+        a.DrawVertexBuffer(vb, fb, C.byref(p), prim, 0, len(data))
+        a.FramebufferDownload(fb)
+        frames.append([x.copy() for x in s.images])
+    assert np.count_nonzero(frames[0][0]) > 4000
+    for x, y in zip(*frames):
+        assert np.array_equal(x.view(np.uint8), y.view(np.uint8))
