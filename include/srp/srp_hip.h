@@ -31,7 +31,8 @@ SRP_EXTERN_C_BEGIN
 
 /** Deferred: draws and clears act on the device copy only; the host arrays
  *  are refreshed by srpFramebufferDownload and pushed by srpFramebufferUpload.
- *  Switching deferred mode on uploads the host arrays once. */
+ *  Switching deferred mode on uploads the host arrays once.  Calls that read
+ *  the host arrays have read them when they return. */
 void srpFramebufferSetDeferred(const SRPFramebuffer* fb, bool deferred);
 void srpFramebufferDownload(const SRPFramebuffer* fb);
 void srpFramebufferUpload(const SRPFramebuffer* fb);

@@ -334,15 +334,16 @@ bool fbOwnArrays(const FbImpl* F)
 	return F->pub.color == F->hColor && F->pub.depth == F->hDepth && F->pub.stencil == F->hStencil;
 }
 
-/* waited: the call does not return before the stream has read the arrays.
- * (A kernel reads them when it runs; a caller that goes on at once keeps the
- * copy calls.) */
-void fbUpload(FbImpl* F, bool waited)
+/* The host arrays to the device copy.  Kernels and copies of pinned memory
+ * read the arrays when the stream reaches them, so a library call that
+ * uploads waits for the stream before it returns (a draw does so in its
+ * download): afterwards the arrays are the caller's, and a clear's, to write. */
+void fbUpload(FbImpl* F)
 {
 	Runtime& R = rt();
 	F->pendColor = F->pendDepth = F->pendStencil = false;  /* the host arrays win */
 	const size_t n = F->pub.size;
-	if (waited && fbOwnArrays(F))
+	if (fbOwnArrays(F))
 	{
 		copyArrays({{F->pub.color, F->pub.depth, F->pub.stencil}, {F->dColor, F->dDepth, F->dStencil}, {n * 4, n * 4, n}},
 		           R.stream);
@@ -351,6 +352,12 @@ void fbUpload(FbImpl* F, bool waited)
 	HIP_CHECK(hipMemcpyAsync(F->dColor, F->pub.color, n * 4, hipMemcpyHostToDevice, R.stream));
 	HIP_CHECK(hipMemcpyAsync(F->dDepth, F->pub.depth, n * 4, hipMemcpyHostToDevice, R.stream));
 	HIP_CHECK(hipMemcpyAsync(F->dStencil, F->pub.stencil, n, hipMemcpyHostToDevice, R.stream));
+}
+
+void fbUploadWait(FbImpl* F)
+{
+	fbUpload(F);
+	HIP_CHECK(hipStreamSynchronize(rt().stream));
 }
 
 void fbDownload(FbImpl* F)
@@ -463,7 +470,7 @@ void framebufferDevice(const SRPFramebuffer* fb, uint32_t** color, float** depth
 	if (F->deferred)
 		fbFlushFills(F);
 	else
-		fbUpload(F, false);
+		fbUploadWait(F);
 	if (color) *color = F->dColor;
 	if (depth) *depth = F->dDepth;
 	if (stencil) *stencil = F->dStencil;
@@ -827,7 +834,7 @@ void srpFramebufferSetDeferred(const SRPFramebuffer* fb, bool deferred)
 	}
 	FbImpl* F = fbImpl(fb);
 	if (deferred && !F->deferred)
-		fbUpload(F, false);
+		fbUploadWait(F);
 	if (!deferred && F->deferred)
 		fbDownload(F);
 	F->deferred = deferred;
@@ -875,8 +882,7 @@ void srpFramebufferUpload(const SRPFramebuffer* fb)
 		message(SRP_MESSAGE_ERROR, SRP_MESSAGE_SEVERITY_HIGH, __func__, "Invalid framebuffer");
 		return;
 	}
-	fbUpload(fbImpl(fb), true);
-	HIP_CHECK(hipStreamSynchronize(rt().stream));
+	fbUploadWait(fbImpl(fb));
 }
 
 void srpFramebufferFillDepth(const SRPFramebuffer* fb, float v)
@@ -1781,7 +1787,7 @@ void drawBuffer(const SRPIndexBuffer* ib, const SRPVertexBuffer* vb, const SRPFr
 	/* a deferred framebuffer's pending fill rides along with the vertex
 	 * stage below (nothing before the rasteriser touches the framebuffer) */
 	if (!F->deferred)
-		fbUpload(F, true);   /* the draw ends in a download */
+		fbUpload(F);   /* the draw ends in a download, which waits */
 	hipEvent_t evDraw = (R.prof(1) || R.prof(3)) ? R.mark() : nullptr;
 	{
 		AsmDraw& AD = *reinterpret_cast<AsmDraw*>((uint8_t*) R.hParams + kAsmDrawOff);
