@@ -797,9 +797,10 @@ void srpFreeFramebuffer(SRPFramebuffer* fb)
 	liveObjects().erase(fb);
 	FbImpl* F = fbImpl(fb);
 	HIP_CHECK(hipStreamSynchronize(rt().stream));
-	HIP_CHECK(hipHostFree(F->pub.color));
-	HIP_CHECK(hipHostFree(F->pub.depth));
-	HIP_CHECK(hipHostFree(F->pub.stencil));
+	/* arrays that a caller put in their place stay the caller's */
+	HIP_CHECK(hipHostFree(F->hColor));
+	HIP_CHECK(hipHostFree(F->hDepth));
+	HIP_CHECK(hipHostFree(F->hStencil));
 	HIP_CHECK(hipFree(F->dColor));
 	HIP_CHECK(hipFree(F->dDepth));
 	HIP_CHECK(hipFree(F->dStencil));

@@ -76,6 +76,34 @@ def test_switch_to_deferred_takes_the_arrays_as_they_are(api, own):
         assert np.array_equal(got[k], want[k]), k
 
 
+@pytest.mark.parametrize("replaced", [("color",), ("depth", "stencil"), ("color", "depth", "stencil")])
+def test_freeing_leaves_the_callers_arrays_alone(api, replaced):
+    """A framebuffer freed with the program's own arrays in place of some or
+    all of its own: they keep what the last download wrote, and the program's
+    next framebuffer works."""
+    w, h = 67, 61
+    mine = {k: np.zeros(w * h * n, np.uint8) for k, n in KINDS}
+    want = {}
+    for turn in range(2):
+        fb = api.NewFramebuffer(w, h)
+        f = api.Fields.from_address(fb)
+        for k in replaced:
+            setattr(f, k, mine[k].ctypes.data)
+        rng = np.random.default_rng(turn)
+        views = host_arrays(api, fb)
+        for k, v in views.items():
+            v[:] = want[k] = rng.integers(0, 256, v.size, dtype=np.uint8)
+        api.FramebufferSetDeferred(fb, True)
+        for v in views.values():
+            v[:] = 0
+        api.FramebufferDownload(fb)
+        del views
+        api.FreeFramebuffer(fb)
+        for k in replaced:
+            assert np.array_equal(mine[k], want[k]), k
+            mine[k][:] = 7
+
+
 def test_staged_passes_keep_the_colours_of_their_call(api):
     """The five passes of a synchronous framebuffer, each cleared (on the
     host) as soon as it is staged."""
