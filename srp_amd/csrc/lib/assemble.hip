@@ -352,21 +352,35 @@ __device__ __forceinline__ bool isSpan(const SrpDrawParams* P, const SrpTri& T)
 }
 
 /* Reserve a span-list entry (one atomic per group of lanes calling
- * together) and fill it: `count` pairs, items item.., record `rec`
- * (0xFFFFFFFF: none). */
+ * together) and fill it: `count` pairs, items item.., record `rec`.  Without
+ * a record (0xFFFFFFFF: a batch's capacity exceeded) the pairs are written
+ * here, empty: the list has as many entries as there are records, and spans
+ * beyond them would leave their items as the buffers happen to be. */
 __device__ void appendSpan(const AsmArgs& A, const SrpDrawParams* P, uint32_t tileBase, uint32_t item, uint32_t count,
                            uint32_t rec)
 {
-	const uint64_t act = __ballot(1);
+	const bool listed = rec != 0xFFFFFFFFu;
+	const uint64_t act = __ballot(listed);
 	const uint32_t lane = __lane_id();
-	const uint32_t leader = (uint32_t) __builtin_ctzll(act);
-	uint32_t at = 0;
-	if (lane == leader)
-		at = atomicAdd(A.spanCount, (uint32_t) __popcll(act));
-	at = (uint32_t) __shfl((int) at, (int) leader) + (uint32_t) __popcll(act & ((1ull << lane) - 1ull));
+	uint32_t at = 0xFFFFFFFFu;
+	if (listed)
+	{
+		const uint32_t leader = (uint32_t) __builtin_ctzll(act);
+		uint32_t first = 0;
+		if (lane == leader)
+			first = atomicAdd(A.spanCount, (uint32_t) __popcll(act));
+		at = __shfl(first, (int) leader) + (uint32_t) __popcll(act & ((1ull << lane) - 1ull));
+	}
 	if (at >= A.spanCap)
 	{
 		atomicOr(A.error, 2u);
+		for (uint32_t k = 0; k < count && (unsigned long long) item + k < A.itemCap; k++)
+		{
+			A.pairKeys[item + k] = tileBase;   /* of any tile */
+			A.pairVals[item + k] = (item + k) | 0x80000000u;
+			A.pairRec[item + k] = 0xFFFFFFFFu;
+			A.pairMask[item + k] = 0ull;
+		}
 		return;
 	}
 	SrpSpan sp;
@@ -1726,7 +1740,7 @@ __global__ __launch_bounds__(128) void k_assemble_points(AsmArgs A)
  * record itself.) */
 __global__ __launch_bounds__(256) void k_expand_spans(const SrpSpan* spans, const SrpTri* tris, const uint32_t* count,
                                                       uint32_t cap, uint32_t* pairKeys, uint32_t* pairVals,
-                                                      uint32_t* pairRec, unsigned long long* pairMask, uint32_t itemCap)
+                                                      uint32_t itemCap)
 {
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t wave = (uint32_t) __builtin_amdgcn_readfirstlane((int) (blockIdx.x * 4u + (threadIdx.x >> 6)));
@@ -1739,21 +1753,6 @@ __global__ __launch_bounds__(256) void k_expand_spans(const SrpSpan* spans, cons
 	for (uint32_t i = wave; i < n; i += nWaves)
 	{
 		const SrpSpan sp = spans[i];
-		if (sp.rec == 0xFFFFFFFFu)
-		{
-			/* no record to find the tiles from: empty pairs of any tile */
-			for (uint32_t k = lane; k < sp.count; k += 64u)
-			{
-				const uint32_t o = sp.item + k;
-				if (o >= itemCap)
-					break;
-				pairKeys[o] = sp.tileBase;
-				pairVals[o] = o | 0x80000000u;
-				pairRec[o] = 0xFFFFFFFFu;
-				pairMask[o] = 0ull;
-			}
-			continue;
-		}
 		const SrpTri* T = tris + sp.rec;
 		SrpSpanScan S;
 		srpSpanScanInit(&S, T->l0, T->dx, T->dy, (int) T->x0, (int) T->y0, (int) T->x1, (int) T->y1);
@@ -1799,7 +1798,7 @@ void launchExpandSpans(const AsmArgs& A, uint32_t blocks, hipStream_t s)
 {
 	if (blocks)
 		hipLaunchKernelGGL(k_expand_spans, dim3(blocks), dim3(256), 0, s, A.spans, A.tris, A.spanCount, A.spanCap,
-		                   A.pairKeys, A.pairVals, A.pairRec, A.pairMask, A.itemCap);
+		                   A.pairKeys, A.pairVals, A.itemCap);
 }
 
 void launchClipped(const AsmArgs& A, bool emit, hipStream_t s, uint32_t clipped, uint32_t clipHint)

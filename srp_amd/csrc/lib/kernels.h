@@ -42,7 +42,7 @@ struct SrpSpan
 {
 	uint32_t item;
 	uint32_t count;
-	uint32_t rec;         /* triangle record, 0xFFFFFFFF: none (capacity exceeded) */
+	uint32_t rec;         /* triangle record */
 	uint32_t tileBase;    /* first tile of the draw's framebuffer */
 	uint32_t tilesX;      /* tiles per framebuffer row */
 	uint32_t shift;       /* log2 of the tile side */
