@@ -136,6 +136,16 @@ constexpr uint32_t OWN_SCAN_MAX_INPUTS = 4096;
  * eight lanes repeat costs more than the scan. */
 constexpr uint32_t ROWS_MAX_INPUTS = 65536;
 
+/* And the least mask box (srpHipSetRasterOptions) of such a draw.  A triangle
+ * larger than the box becomes a span, whose tile rows all eight lanes walk;
+ * with a small box that is most triangles, and the few that are masked are
+ * quick to scan.  Frames at 1920x1080, us with a lane and with eight lanes a
+ * triangle: 60,000 of some 6 pixels, box 0 to 4 205 / 350, box 8 197 / 316,
+ * 16 201 / 177, 24 227 / 159; 20,000 of some 12 pixels, box 8 179 / 208, 16
+ * 217 / 199, 24 266 / 170.  (Of 60,000 with some 12 or 24 pixels a lane is
+ * better up to a box of 16 and 24: 292 / 370, 506 / 547.) */
+constexpr uint32_t ROWS_MIN_MASK_BOX = 16;
+
 /* kind: 0 triangles, 1 lines, 2 points.  clipped: how many triangles the
  * counting pass listed for clipping, when the caller knows it (0 skips the
  * clipped-triangle kernel); with kClipUnknown its grid is sized from

@@ -1863,7 +1863,8 @@ void drawBuffer(const SRPIndexBuffer* ib, const SRPVertexBuffer* vb, const SRPFr
 	A.clipCount = totals + 4;
 	A.spanCount = totals + 6;   /* counting pass: how many spans */
 	A.recCap = A.itemCap = A.genCap = 0xFFFFFFFFu;
-	if (kind == 0 && S.polygonMode == SRP_POLYGON_MODE_FILL && R.tile == 8 && nIn <= ROWS_MAX_INPUTS)
+	if (kind == 0 && S.polygonMode == SRP_POLYGON_MODE_FILL && R.tile == 8 && R.maskBox >= ROWS_MIN_MASK_BOX &&
+	    nIn <= ROWS_MAX_INPUTS)
 		A.rows = (uint32_t) nIn;
 	D.kind = kind;
 	D.backend = (kind == 0) ? (int) S.polygonMode : (kind == 1 ? 1 : 2);  /* 0 tiles, 1 lines, 2 points */
