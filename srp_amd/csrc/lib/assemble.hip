@@ -341,8 +341,8 @@ __device__ __forceinline__ uint32_t binTriangle(const SrpDrawParams* P, const Sr
 	return spanTiles(P, T);
 }
 
-/* True when binTriangle gives T one unmasked entry per tile of its box
- * (a span) rather than exact masks. */
+/* True when binTriangle gives T entries without masks (a span: the tiles its
+ * edges let it reach) rather than exact ones. */
 __device__ __forceinline__ bool isSpan(const SrpDrawParams* P, const SrpTri& T)
 {
 	if (T.x1 <= T.x0 || T.y1 <= T.y0)
@@ -1505,7 +1505,12 @@ struct LineWork
  * walking its own line takes as long as the wave's longest; here the lanes
  * take LINE_CHUNK samples at a time, of any line, the DDA's sums up to a
  * chunk's first sample replayed exactly (srpReplay): 100,000 lines
- * (6.06 M samples) over 1920x1080 in 112 us, 230 with a lane each. */
+ * (6.06 M samples) over 1920x1080 in 112 us, 230 with a lane each.
+ * Sixteen: fewer samples replay more sums, more leave a wave's last lines to
+ * few lanes and write further apart.  Emitting pass, us with 8, 16 and 32,
+ * lines at 1920x1080 with lognormal lengths: 100,000 of some 20 pixels 47, 49,
+ * 54; of 60 109, 113, 146; of 200 315, 307, 543; 2,000 of 60 83, 59, 55; of
+ * 600 626, 430, 327. */
 constexpr int LINE_CHUNK = 16;
 __device__ __forceinline__ void emitWaveLines(const AsmArgs& A, const SrpDrawParams* P, const LineWork& w)
 {
@@ -1805,9 +1810,14 @@ void launchClipped(const AsmArgs& A, bool emit, hipStream_t s, uint32_t clipped,
 {
 	const uint32_t blocks = A.nBlocks;
 	if (!blocks) return;
-	/* at most 8,192 blocks: what the chip holds at once (2,048) left it idle
-	 * at the end, some groups having much more to do (the figures above: 707
-	 * and 867 us, 676 and 714 so) */
+	/* The clip list's length is on the device; the grid strides over it, 8
+	 * triangles a block (groups of CLIP_GROUP lanes).  A known count gets a
+	 * group a triangle; an unknown one is sized from the caller's hint (the
+	 * count of a similar earlier draw, a quarter more), at least 256 blocks,
+	 * and at most a group for every input (the main grid has 128 inputs a
+	 * block).  Both at most 8,192 blocks: what the chip holds at once (2,048)
+	 * left it idle at the end, some groups having much more to do (the clipped
+	 * of 500,000 triangles over 1920x1080: 707 and 867 us, 676 and 714 so). */
 	uint32_t clipBlocks;
 	if (clipped != kClipUnknown)
 	{
@@ -1818,9 +1828,8 @@ void launchClipped(const AsmArgs& A, bool emit, hipStream_t s, uint32_t clipped,
 	{
 		const uint64_t want = ((uint64_t) clipHint + clipHint / 4u + 7u) / 8u;
 		clipBlocks = (uint32_t) (want < 256u ? 256u : (want > 8192u ? 8192u : want));
-		/* (a group per triangle of a draw that clips much of its few
-		 * inputs: limited to the main grid, 2,000 triangles of which half
-		 * are clipped took eight rounds, 117 + 144 us; 52 + 36 with a group each) */
+		/* (limited to the main grid's blocks, 2,000 triangles of which half
+		 * are clipped took eight rounds, 117 + 144 us; 52 + 36 so) */
 		clipBlocks = (uint64_t) clipBlocks < 16ull * blocks ? clipBlocks : 16u * blocks;
 	}
 	if (!clipBlocks)
@@ -1837,14 +1846,7 @@ void launchAssemble(const AsmArgs& A, int kind, bool emit, hipStream_t s, uint32
 	{
 		case 0:
 		{
-			/* The clip list's length is on the device; a grid strides over
-			 * it, 8 triangles per block (groups of CLIP_GROUP lanes).  A
-			 * known count gets a group per triangle (up to 2048 blocks); an
-			 * unknown one is sized from the caller's hint (the count of a
-			 * similar earlier draw, a quarter more), at least 256 blocks
-			 * (the empty grid of a draw that clips nothing still costs its
-			 * dispatch), and never more blocks than the draw's main
-			 * assembly grid (which has 128 inputs a block) can list. */
+			/* (the clipped triangles' grid: launchClipped) */
 			if (A.rows)
 			{
 				const uint32_t rb = (uint32_t) (((uint64_t) A.rows * ROW_GROUP + 127u) / 128u);

@@ -294,9 +294,10 @@ void scanExclusiveMulti(uint32_t* base, size_t stride, int nArrays, size_t n, ui
 
 /* Tile ranges of a list sorted by tile: [start, end) per tile; tiles that
  * received nothing keep start == end == 0 (set by the caller's fill).  A
- * thread takes EACH items: four from one load where the list is long (92 M
- * items: 188 us with one each, 96 with four), one where it is short and the
- * threads few (350 k items: 2.6 and 3.7 us). */
+ * thread takes EACH items: four from one load where the list is long, one
+ * where it is short and the threads few.  us with one and with four, traced:
+ * 37 k items 2.2 and 3.4, 350 k 2.6 and 3.7, 0.75 M and 1.4 M 5.3 and 5.3,
+ * 3.0 M 6.6 and 5.8, 7.4 M 11.7 and 9.1, 18 M 24 and 17, 74 M 111 and 69. */
 constexpr size_t TB_LONG_FROM = (size_t) 4 << 20;
 
 template <int EACH>
@@ -350,7 +351,12 @@ constexpr int RS_CHUNK = 1024;   /* items per block: more blocks than CUs for th
 /* A sort of more than RS_LONG_FROM items takes whole rounds of
  * RS_LONG_ROUND items a block (k_radix_scatter_long), some RS_LONG_BLOCKS
  * blocks of at most RS_LONG_CHUNK: enough to fill the chip several times
- * over, and few enough digit counts to scan. */
+ * over, and few enough digit counts to scan.  Kernel time of two passes over
+ * the tile pairs of large triangles, us with the short sort's blocks and with
+ * these: 1.05 M items 73 and 51, 1.5 M 88 and 53, 2 M 110 and 55, 4 M 184 and
+ * 84, 8 M 345 and 135, 40 M 1,549 and 570.  (300 k: 36 and 44, fused passes
+ * and not.)  1,024 and 4,096 blocks: within the noise up to 8 M, 245 and 236
+ * against 221 at 16 M, 587 and 563 against 570 at 40 M. */
 constexpr int RS_LONG_ROUND = 4096;
 constexpr int RS_LONG_CHUNK = 32768;
 constexpr int RS_LONG_BLOCKS = 2048;
@@ -688,8 +694,9 @@ __global__ __launch_bounds__(RS_THREADS) void k_radix_scatter_long(const uint32_
 				valsOut[dst] = sortedVal[p];
 			}
 		}
-		/* the next round's writes of cnt follow this round's reads of it by
-		 * two barriers, those of the sorted items by three */
+		/* the next round's first writes of cnt are each wave's to its own
+		 * row, which since the last barrier only that wave reads; its writes
+		 * of the sorted items follow this round's reads by three barriers */
 	}
 }
 
